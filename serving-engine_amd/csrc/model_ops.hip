@@ -1036,6 +1036,52 @@ rmsnorm_rows_kernel(const f16* x, const f16* w, f16* out, int dim, float eps) {
             static_cast<f16>(static_cast<float>(xr[k]) * rs * static_cast<float>(w[k]));
 }
 
+// The same for rows that fit the registers of WPR waves (dim % 8 == 0, NV
+// 16-byte chunks a lane): HBM-bound, every row read once with 16-byte loads.
+// One wave per row up to 4096 columns (no barrier; four rows a workgroup),
+// four beyond.  1999 x 2048: 8.9 us with 2-byte accesses, 5.2 us (3.2 TB/s) now.
+template <int WPR, int NV>
+__global__ void __launch_bounds__(256)
+rmsnorm_vec_kernel(const f16* x, const f16* w, f16* out, int64_t rows, int dim, float eps) {
+    __shared__ float part[4];
+    const int lane = static_cast<int>(threadIdx.x) & (WPR * kWave - 1);
+    const int64_t r = blockIdx.x * (int64_t)(4 / WPR) + threadIdx.x / (WPR * kWave);
+    if (WPR == 1 && r >= rows) return;
+    const f16* xr = x + r * dim;
+    const int chunks = dim / 8;
+    half8 xv[NV], wv[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = lane + j * WPR * kWave;
+        xv[j] = c < chunks ? load_half8(xr + 8 * c) : half8{};
+        wv[j] = c < chunks ? load_half8(w + 8 * c) : half8{};
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float v = static_cast<float>(xv[j][e]);
+            ss = fmaf(v, v, ss);
+        }
+    ss = wave_sum_fast(ss);
+    if constexpr (WPR == 4) {
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = part[0] + part[1] + part[2] + part[3];
+    }
+    const float rs = 1.f / sqrtf(ss / static_cast<float>(dim) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = lane + j * WPR * kWave;
+        half8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            o[e] = static_cast<f16>(static_cast<float>(xv[j][e]) * rs * static_cast<float>(wv[j][e]));
+        if (c < chunks) store_half8(out + r * dim + 8 * c, o);
+    }
+}
+
 // RoPE in place on token-major q [S][Hq][D] and k [S][Hkv][D] (reference
 // apply_rope, kernels.h:57-70): one thread per rotation pair.
 __global__ void rope_kernel(f16* q, f16* k, int64_t S, int Hq, int Hkv, int D, int start_pos,
@@ -1092,6 +1138,72 @@ __global__ void split_qkv_rope_kernel(const f16* qkv, int64_t S, int Hq, int Hkv
     }
 }
 
+// The same for D % 16 == 0 and 16-byte aligned tensors.  A workgroup takes TB
+// tokens and computes each token's D/2 rotations once, into LDS, for all of
+// its heads (one powf, cosf and sinf per pair and head cost more than the
+// memory traffic); a thread then rotates 8 pairs at a time with 16-byte
+// accesses, its loads issued before the rotations.  HBM-bound.  1999 tokens of
+// 32 + 2 * 4 heads of 64: 21.9 us one pair per thread, 7.3 us now.
+constexpr int kRopePairs = 128;   // rotations per workgroup: TB = max(1, 128 / (D/2))
+
+__global__ void __launch_bounds__(256)
+split_qkv_rope_vec_kernel(const f16* qkv, int64_t S, int Hq, int Hkv, int D, int start_pos,
+                          const int32_t* positions, float theta, f16* q, f16* k, f16* v, int TB) {
+    constexpr int U = 3;              // pair chunks of a thread in flight
+    __shared__ float2 cs[256];        // [TB][D/2], D/2 <= 256
+    const int half = D / 2, H = Hq + 2 * Hkv;
+    const int cph = half / 8;         // 8-pair chunks per head
+    const int per_tok = H * cph;
+    const int64_t s0 = (int64_t)blockIdx.x * TB;
+    const int nt = static_cast<int>(min((int64_t)TB, S - s0));
+    const int items = nt * per_tok;
+    for (int base = 0; base < items; base += 256 * U) {
+        half8 a[U], b[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int it = base + 256 * u + static_cast<int>(threadIdx.x);
+            if (it < items) {
+                const f16* src = qkv + (s0 * H + it / cph) * D + 8 * (it % cph);
+                a[u] = load_half8(src);
+                b[u] = load_half8(src + half);
+            }
+        }
+        if (base == 0) {
+            const int t = static_cast<int>(threadIdx.x);
+            if (t < nt * half) {
+                const int64_t s = s0 + t / half;
+                const int pos = positions ? max(positions[s], 0) : static_cast<int>(start_pos + s);
+                rope_cs(pos, t % half, D, theta, cs[t].x, cs[t].y);
+            }
+            lds_barrier();
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int it = base + 256 * u + static_cast<int>(threadIdx.x);
+            if (it >= items) break;
+            const int c = it % cph, sh = it / cph;
+            const int h = sh % H, tt = sh / H;
+            const int64_t s = s0 + tt;
+            half8 o1 = a[u], o2 = b[u];
+            f16* dst;
+            if (h < Hq + Hkv) {
+                const float2* r = cs + tt * half + 8 * c;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float x1 = static_cast<float>(a[u][e]), x2 = static_cast<float>(b[u][e]);
+                    o1[e] = static_cast<f16>(x1 * r[e].x - x2 * r[e].y);
+                    o2[e] = static_cast<f16>(x2 * r[e].x + x1 * r[e].y);
+                }
+                dst = h < Hq ? q + (s * Hq + h) * D : k + (s * Hkv + (h - Hq)) * D;
+            } else {
+                dst = v + (s * Hkv + (h - Hq - Hkv)) * D;
+            }
+            store_half8(dst + 8 * c, o1);
+            store_half8(dst + 8 * c + half, o2);
+        }
+    }
+}
+
 // SwiGLU over rows of a fused [gate | up] buffer [rows][2n] -> out [rows][n];
 // with row stride 0 and n = count this is the reference's flat swiglu.
 __global__ void swiglu_kernel(const f16* gate, const f16* up, int64_t in_stride, f16* out,
@@ -1106,6 +1218,23 @@ __global__ void swiglu_kernel(const f16* gate, const f16* up, int64_t in_stride,
     }
 }
 
+// The same, 8 columns a thread (n % 8 == 0, 16-byte aligned tensors): HBM-bound.
+// 1999 x 5632: 21.8 us with 2-byte accesses, 15.9 us (4.2 TB/s) now.
+__global__ void __launch_bounds__(256)
+swiglu_vec_kernel(const f16* gate, const f16* up, int64_t in_stride, f16* out, uint32_t chunks,
+                  uint32_t row_chunks) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= chunks) return;
+    const uint32_t r = t / row_chunks, c = t % row_chunks;
+    const int64_t in = r * in_stride + 8 * (int64_t)c;
+    const half8 g = load_half8(gate + in), u = load_half8(up + in);
+    half8 o;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        o[e] = static_cast<f16>(silu_mul(static_cast<float>(g[e]), static_cast<float>(u[e])));
+    store_half8(out + 8 * (int64_t)t, o);
+}
+
 // Embedding lookup: out[i][:] = table[ids[i]][:] (ids device int32; ids
 // outside [0, vocab) give zero rows).
 __global__ void embedding_kernel(const int32_t* ids, const f16* table, f16* out, int64_t n,
@@ -1114,6 +1243,20 @@ __global__ void embedding_kernel(const int32_t* ids, const f16* table, f16* out,
     const int64_t id = ids[i];
     for (int64_t k = threadIdx.x; k < hidden; k += blockDim.x)
         out[i * hidden + k] = (id >= 0 && id < vocab) ? table[id * hidden + k] : static_cast<f16>(0.f);
+}
+
+// The same, 8 columns a thread (hidden % 8 == 0, 16-byte aligned tensors), a
+// wave's worth of columns after another so that short rows fill the
+// workgroups too.  1999 rows of 2048: 7.2 us with 2-byte accesses, 4.8 us now.
+__global__ void __launch_bounds__(256)
+embedding_vec_kernel(const int32_t* ids, const f16* table, f16* out, uint32_t chunks,
+                     uint32_t row_chunks, int64_t vocab) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= chunks) return;
+    const uint32_t i = t / row_chunks, c = t % row_chunks;
+    const int64_t id = ids[i];
+    const f16* src = table + (id * row_chunks + c) * 8;
+    store_half8(out + 8 * (int64_t)t, id >= 0 && id < vocab ? load_half8(src) : half8{});
 }
 
 // The same rows into row-tiled activations (hidden % 32 == 0, 16-byte
@@ -1679,10 +1822,34 @@ extern "C" int kvhp_rmsnorm(const void* x, const void* weight, void* out, int64_
     if (rows <= 0) return KVHP_OK;
     KVHP_REQUIRE(x && weight && out && dim > 0 && dim <= (1 << 24), KVHP_ERR_INVALID,
                  "rmsnorm: bad arguments");
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const f16*>(x),
-                       static_cast<const f16*>(weight), static_cast<f16*>(out),
-                       static_cast<int>(dim), eps);
+    const f16* xp = static_cast<const f16*>(x);
+    const f16* wp = static_cast<const f16*>(weight);
+    f16* op = static_cast<f16*>(out);
+    const int n = static_cast<int>(dim);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    // Whole rows in registers where the chunks are aligned; dims past 16384
+    // and odd ones keep the looping kernel.
+    if (dim % 8 == 0 && dim <= 16384 && rows <= 0x7fffffff && aligned16(x) && aligned16(weight) &&
+        aligned16(out)) {
+        auto launch = [&](auto kern, int rows_per_wg) {
+            const int64_t g = (rows + rows_per_wg - 1) / rows_per_wg;
+            hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(g)), dim3(256), 0, s, xp, wp, op,
+                               rows, n, eps);
+        };
+        if (dim <= 1024)
+            launch(rmsnorm_vec_kernel<1, 2>, 4);
+        else if (dim <= 2048)
+            launch(rmsnorm_vec_kernel<1, 4>, 4);
+        else if (dim <= 4096)
+            launch(rmsnorm_vec_kernel<1, 8>, 4);
+        else if (dim <= 8192)
+            launch(rmsnorm_vec_kernel<4, 4>, 1);
+        else
+            launch(rmsnorm_vec_kernel<4, 8>, 1);
+        return check_launch("rmsnorm");
+    }
+    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, s,
+                       xp, wp, op, n, eps);
     return check_launch("rmsnorm");
 }
 
@@ -1703,6 +1870,40 @@ extern "C" int kvhp_apply_rope(void* q, void* k, int64_t seq_len, int64_t num_q_
     return check_launch("apply_rope");
 }
 
+namespace {
+void launch_split_qkv_rope(const f16* qkv, int64_t rows, int Hq, int Hkv, int D, int start_pos,
+                           const int32_t* positions, float theta, f16* q, f16* k, f16* v,
+                           hipStream_t s) {
+    const int64_t H = (int64_t)Hq + 2 * (int64_t)Hkv, half = D / 2;
+    // the vector kernel: whole 16-byte chunks of both halves, the rotations of
+    // a token in its LDS table, 32-bit item counts
+    if (D % 16 == 0 && half <= 256 && H * half < (1 << 22) && rows <= 0x7fffffff &&
+        aligned16(qkv) && aligned16(q) && aligned16(k) && aligned16(v)) {
+        const int TB = static_cast<int>(std::max<int64_t>(1, kRopePairs / half));
+        hipLaunchKernelGGL(split_qkv_rope_vec_kernel,
+                           dim3(static_cast<unsigned>((rows + TB - 1) / TB)), dim3(256), 0, s,
+                           qkv, rows, Hq, Hkv, D, start_pos, positions, theta, q, k, v, TB);
+        return;
+    }
+    hipLaunchKernelGGL(split_qkv_rope_kernel, dim3(grid_for(rows * H * half, 256)), dim3(256), 0,
+                       s, qkv, rows, Hq, Hkv, D, start_pos, positions, theta, q, k, v);
+}
+
+// SwiGLU over rows; the vector kernel for aligned 8-column chunks.
+void launch_swiglu(const f16* gate, const f16* up, int64_t in_stride, f16* out, int64_t rows,
+                   int64_t n, hipStream_t s) {
+    const int64_t chunks = rows * (n / 8);
+    if (n % 8 == 0 && chunks < ((int64_t)1 << 31) && aligned16(gate) && aligned16(up) &&
+        aligned16(out))
+        hipLaunchKernelGGL(swiglu_vec_kernel, dim3(static_cast<unsigned>((chunks + 255) / 256)),
+                           dim3(256), 0, s, gate, up, in_stride, out,
+                           static_cast<uint32_t>(chunks), static_cast<uint32_t>(n / 8));
+    else
+        hipLaunchKernelGGL(swiglu_kernel, dim3(grid_for(rows * n, 256)), dim3(256), 0, s, gate,
+                           up, in_stride, out, rows, n);
+}
+}  // namespace
+
 extern "C" int kvhp_split_qkv_rope(const void* qkv, int64_t seq_len, int num_q_heads,
                                    int num_kv_heads, int head_dim, int64_t start_pos,
                                    float rope_theta, void* q, void* k, void* v, void* stream) {
@@ -1711,12 +1912,10 @@ extern "C" int kvhp_split_qkv_rope(const void* qkv, int64_t seq_len, int num_q_h
     KVHP_REQUIRE(qkv && q && k && v && head_dim > 0 && head_dim % 2 == 0 && num_q_heads > 0 &&
                      num_kv_heads > 0,
                  KVHP_ERR_INVALID, "split_qkv_rope: bad arguments");
-    const int64_t pairs = seq_len * (num_q_heads + 2 * num_kv_heads) * (head_dim / 2);
-    hipLaunchKernelGGL(split_qkv_rope_kernel, dim3(grid_for(pairs, 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const f16*>(qkv), seq_len,
-                       num_q_heads, num_kv_heads, head_dim, static_cast<int>(start_pos),
-                       static_cast<const int32_t*>(nullptr), rope_theta, static_cast<f16*>(q),
-                       static_cast<f16*>(k), static_cast<f16*>(v));
+    launch_split_qkv_rope(static_cast<const f16*>(qkv), seq_len, num_q_heads, num_kv_heads,
+                          head_dim, static_cast<int>(start_pos), nullptr, rope_theta,
+                          static_cast<f16*>(q), static_cast<f16*>(k), static_cast<f16*>(v),
+                          static_cast<hipStream_t>(stream));
     return check_launch("split_qkv_rope");
 }
 
@@ -1729,11 +1928,9 @@ extern "C" int kvhp_split_qkv_rope_rows(const void* qkv, int64_t rows, int num_q
     KVHP_REQUIRE(qkv && positions && q && k && v && head_dim > 0 && head_dim % 2 == 0 &&
                      num_q_heads > 0 && num_kv_heads > 0,
                  KVHP_ERR_INVALID, "split_qkv_rope_rows: bad arguments");
-    const int64_t pairs = rows * (num_q_heads + 2 * num_kv_heads) * (head_dim / 2);
-    hipLaunchKernelGGL(split_qkv_rope_kernel, dim3(grid_for(pairs, 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const f16*>(qkv), rows,
-                       num_q_heads, num_kv_heads, head_dim, 0, positions, rope_theta,
-                       static_cast<f16*>(q), static_cast<f16*>(k), static_cast<f16*>(v));
+    launch_split_qkv_rope(static_cast<const f16*>(qkv), rows, num_q_heads, num_kv_heads, head_dim,
+                          0, positions, rope_theta, static_cast<f16*>(q), static_cast<f16*>(k),
+                          static_cast<f16*>(v), static_cast<hipStream_t>(stream));
     return check_launch("split_qkv_rope_rows");
 }
 
@@ -1742,10 +1939,8 @@ extern "C" int kvhp_swiglu(const void* gate, const void* up, void* out, int64_t 
     clear_error();
     if (count <= 0) return KVHP_OK;
     KVHP_REQUIRE(gate && up && out, KVHP_ERR_INVALID, "swiglu: null pointer");
-    hipLaunchKernelGGL(swiglu_kernel, dim3(grid_for(count, 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), static_cast<const f16*>(gate),
-                       static_cast<const f16*>(up), (int64_t)0, static_cast<f16*>(out),
-                       (int64_t)1, count);
+    launch_swiglu(static_cast<const f16*>(gate), static_cast<const f16*>(up), 0,
+                  static_cast<f16*>(out), 1, count, static_cast<hipStream_t>(stream));
     return check_launch("swiglu");
 }
 
@@ -1755,9 +1950,8 @@ extern "C" int kvhp_swiglu_rows(const void* gate_up, void* out, int64_t rows, in
     if (rows <= 0 || n <= 0) return KVHP_OK;
     KVHP_REQUIRE(gate_up && out, KVHP_ERR_INVALID, "swiglu_rows: null pointer");
     const f16* g = static_cast<const f16*>(gate_up);
-    hipLaunchKernelGGL(swiglu_kernel, dim3(grid_for(rows * n, 256)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), g, g + n, 2 * n, static_cast<f16*>(out),
-                       rows, n);
+    launch_swiglu(g, g + n, 2 * n, static_cast<f16*>(out), rows, n,
+                  static_cast<hipStream_t>(stream));
     return check_launch("swiglu_rows");
 }
 
@@ -1767,6 +1961,15 @@ extern "C" int kvhp_embedding(const int32_t* token_ids, const void* table, void*
     if (n <= 0) return KVHP_OK;
     KVHP_REQUIRE(token_ids && table && out && hidden > 0 && vocab > 0, KVHP_ERR_INVALID,
                  "embedding: bad arguments");
+    if (hidden % 8 == 0 && n <= 0x7fffffff && hidden / 8 < (1 << 30) &&
+        n * (hidden / 8) < ((int64_t)1 << 31) && aligned16(table) && aligned16(out)) {
+        const uint32_t chunks = static_cast<uint32_t>(n * (hidden / 8));
+        hipLaunchKernelGGL(embedding_vec_kernel, dim3((chunks + 255) / 256), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), token_ids,
+                           static_cast<const f16*>(table), static_cast<f16*>(out), chunks,
+                           static_cast<uint32_t>(hidden / 8), vocab);
+        return check_launch("embedding");
+    }
     hipLaunchKernelGGL(embedding_kernel, dim3(static_cast<unsigned>(n)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), token_ids,
                        static_cast<const f16*>(table), static_cast<f16*>(out), n, hidden, vocab);
