@@ -18,7 +18,9 @@
 //             projection (rope.cu:8-57 then kv_cache.cu:8-36: q/k rounded to
 //             fp16, rotated in fp32, rounded again; k and v written into their
 //             16-token pages at position seq_len - 1).
-// A generic one-wave-per-row kernel covers shapes the fast one does not.
+// K of whole 16-byte chunks other than those two is covered by chunks masked
+// past K or by slabs; a generic one-wave-per-row kernel covers other K and
+// unaligned operands.
 //
 // Prefill uses library GEMMs (rocBLAS) for the projections; the row-wise
 // RMSNorm, the RoPE that also splits the fused QKV output, and SwiGLU over
@@ -82,10 +84,16 @@ __device__ __forceinline__ void rope_cs(int pos, int i, int D, float theta, floa
     s = sinf(ang);
 }
 
-// Fast GEMV: K == 512*KC, RW rows per wave (one wave per workgroup).
-template <int KC, int RW, int EPI, bool RMS>
+// How a wave covers K with 16-byte chunks per lane: exactly KC of them
+// (K == 512*KC), up to KC with the chunks past K zero (K % 8 == 0), or slabs
+// of KC one after another (any larger K % 8 == 0).
+enum Cover : int { kExact = 0, kTail = 1, kSlabs = 2 };
+
+// Fast GEMV, RW rows per wave (one wave per workgroup).
+template <int KC, int RW, int EPI, bool RMS, int COVER = kExact>
 __global__ void __launch_bounds__(kWave) gemv_kernel(const GemvArgs a) {
     const int lane = threadIdx.x;
+    const int nchunk = a.K / 8;
 
     // The rows of this wave.
     int row[RW];
@@ -125,19 +133,44 @@ __global__ void __launch_bounds__(kWave) gemv_kernel(const GemvArgs a) {
     // RMSNorm waits only for them and runs while the weights stream in
     // (behind the weights it waited for every weight load: QKV 4.25 vs
     // 3.58 us without the norm, in a HIP graph).
-    half8 xr[KC], nw[KC];
+    // Slabs load and multiply one slab at a time (below); several waves per SIMD
+    // keep the memory busy meanwhile.
+    half8 xr[KC], nw[KC], wr[RW][KC];
+    auto chunk = [&](const f16* p, int j, bool stream) {
+        if (COVER != kExact && 64 * j + lane >= nchunk) return half8{};
+        p += 512 * j + 8 * lane;
+        return stream ? load_half8_stream(p) : load_half8(p);
+    };
+    auto load_x = [&](int j0) {
 #pragma unroll
-    for (int j = 0; j < KC; ++j) {
-        xr[j] = load_half8(a.x + 512 * j + 8 * lane);
-        if constexpr (RMS) nw[j] = load_half8(a.norm_w + 512 * j + 8 * lane);
+        for (int j = 0; j < KC; ++j) {
+            xr[j] = chunk(a.x, j0 + j, false);
+            if constexpr (RMS) nw[j] = chunk(a.norm_w, j0 + j, false);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // keep them ahead of the weights
+    };
+    auto load_w = [&](int j0) {
+#pragma unroll
+        for (int i = 0; i < RW; ++i)
+#pragma unroll
+            for (int j = 0; j < KC; ++j) wr[i][j] = chunk(a.W + (int64_t)row[i] * a.K, j0 + j, true);
+    };
+    if constexpr (COVER == kExact) {
+#pragma unroll
+        for (int j = 0; j < KC; ++j) {
+            xr[j] = load_half8(a.x + 512 * j + 8 * lane);
+            if constexpr (RMS) nw[j] = load_half8(a.norm_w + 512 * j + 8 * lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // keep them ahead of the weights
+#pragma unroll
+        for (int i = 0; i < RW; ++i)
+#pragma unroll
+            for (int j = 0; j < KC; ++j)
+                wr[i][j] = load_half8_stream(a.W + (int64_t)row[i] * a.K + 512 * j + 8 * lane);
+    } else if constexpr (COVER == kTail) {
+        load_x(0);
+        load_w(0);
     }
-    __builtin_amdgcn_sched_barrier(0);   // keep them ahead of the weights
-    half8 wr[RW][KC];
-#pragma unroll
-    for (int i = 0; i < RW; ++i)
-#pragma unroll
-        for (int j = 0; j < KC; ++j)
-            wr[i][j] = load_half8_stream(a.W + (int64_t)row[i] * a.K + 512 * j + 8 * lane);
     // The epilogue's own reads (residual row, write position and its page)
     // ride the same round trip.
     float rv = 0.f;
@@ -164,31 +197,71 @@ __global__ void __launch_bounds__(kWave) gemv_kernel(const GemvArgs a) {
             asm volatile("" ::"v"(rc), "v"(rs));
         }
     }
-    if constexpr (RMS) {
+    float acc[RW];
+    if constexpr (COVER == kSlabs) {
+        const int groups = (nchunk + 63) / 64;
         float ss = 0.f;
+        if constexpr (RMS) {
+            for (int j0 = 0; j0 < groups; j0 += KC) {
+                load_x(j0);
 #pragma unroll
-        for (int j = 0; j < KC; ++j)
+                for (int j = 0; j < KC; ++j)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v = static_cast<float>(xr[j][e]);
-                ss = fmaf(v, v, ss);
+                    for (int e = 0; e < 8; ++e) {
+                        const float v = static_cast<float>(xr[j][e]);
+                        ss = fmaf(v, v, ss);
+                    }
             }
-        ss = wave_sum_fast(ss);
+            ss = wave_sum_fast(ss);
+        }
         const float rs = 1.f / sqrtf(ss / static_cast<float>(a.K) + a.eps);
 #pragma unroll
-        for (int j = 0; j < KC; ++j)
+        for (int i = 0; i < RW; ++i) acc[i] = 0.f;
+        for (int j0 = 0; j0 < groups; j0 += KC) {
+            load_x(j0);
+            load_w(j0);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (RMS) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                xr[j][e] = static_cast<f16>(static_cast<float>(xr[j][e]) * rs *
-                                            static_cast<float>(nw[j][e]));
-    }
-    float acc[RW];
+                for (int j = 0; j < KC; ++j)
 #pragma unroll
-    for (int i = 0; i < RW; ++i) {
-        acc[i] = 0.f;
+                    for (int e = 0; e < 8; ++e)
+                        xr[j][e] = static_cast<f16>(static_cast<float>(xr[j][e]) * rs *
+                                                    static_cast<float>(nw[j][e]));
+            }
 #pragma unroll
-        for (int j = 0; j < KC; ++j) acc[i] = dot8(wr[i][j], xr[j], acc[i]);
-        acc[i] = wave_sum_fast(acc[i]);
+            for (int i = 0; i < RW; ++i)
+#pragma unroll
+                for (int j = 0; j < KC; ++j) acc[i] = dot8(wr[i][j], xr[j], acc[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < RW; ++i) acc[i] = wave_sum_fast(acc[i]);
+    } else {
+        if constexpr (RMS) {
+            float ss = 0.f;
+#pragma unroll
+            for (int j = 0; j < KC; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float v = static_cast<float>(xr[j][e]);
+                    ss = fmaf(v, v, ss);
+                }
+            ss = wave_sum_fast(ss);
+            const float rs = 1.f / sqrtf(ss / static_cast<float>(a.K) + a.eps);
+#pragma unroll
+            for (int j = 0; j < KC; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    xr[j][e] = static_cast<f16>(static_cast<float>(xr[j][e]) * rs *
+                                                static_cast<float>(nw[j][e]));
+        }
+#pragma unroll
+        for (int i = 0; i < RW; ++i) {
+            acc[i] = 0.f;
+#pragma unroll
+            for (int j = 0; j < KC; ++j) acc[i] = dot8(wr[i][j], xr[j], acc[i]);
+            acc[i] = wave_sum_fast(acc[i]);
+        }
     }
 
     // Lane i (< RW) finishes row i (every lane holds every sum).
@@ -344,23 +417,44 @@ int launch_gemv(const GemvArgs& a, hipStream_t s) {
     else
         units = a.N;
     const bool xa = aligned16(a.x) && aligned16(a.W) && (!RMS || aligned16(a.norm_w));
+    auto grid_of = [&](int RW) {
+        if constexpr (EPI == kEpiQKV)
+            return (a.Hq + 2 * a.Hkv) * (a.D / RW);
+        else if constexpr (EPI == kEpiSwiglu)
+            return (a.N + RW / 2 - 1) / (RW / 2);
+        else
+            return (a.N + RW - 1) / RW;
+    };
     // Two rows per wave: the decode GEMVs are latency-bound, and more, smaller
     // waves in flight beat fewer that each stream more rows (measured on the
     // config-5 step: 1448 tok/s at 2 rows, 1430 at 4, 1376 at 8).
+    constexpr int RW = 2;
+    auto launch = [&](auto kern, int rw) {
+        hipLaunchKernelGGL(kern, dim3(grid_of(rw)), dim3(kWave), 0, s, a);
+    };
     if (xa && a.K == 2048) {
-        constexpr int RW = 2;
-        int grid;
-        if constexpr (EPI == kEpiQKV)
-            grid = (a.Hq + 2 * a.Hkv) * (a.D / RW);
-        else if constexpr (EPI == kEpiSwiglu)
-            grid = (a.N + RW / 2 - 1) / (RW / 2);
+        launch(gemv_kernel<4, RW, EPI, RMS>, RW);
+    } else if (xa && a.K % 8 == 0) {
+        // Any other K of whole 16-byte chunks: the row in registers up to 4096
+        // columns (at most 152 VGPRs), slabs of 4096 beyond.  Against the
+        // element-wise kernel at hidden 896, FFN 4864: LM head (32000 x 896)
+        // 9.3 vs 37.4 us (6.2 TB/s), gate/up 4.2 vs 15.5, down 3.7 vs 24.8,
+        // QKV 2.7 vs 14.7, o 2.4 vs 5.6 us; at hidden 4096, FFN 11264: head
+        // 43.1 us (6.1 TB/s), gate/up 32.4, down 17.2 us (5.4 TB/s).
+        if constexpr (EPI != kEpiQKV && EPI != kEpiSwiglu) {
+            if (a.K == 5632) {
+                launch(gemv_kernel<11, RW, EPI, RMS>, RW);
+                return check_launch("gemv");
+            }
+        }
+        if (a.K <= 1024)
+            launch(gemv_kernel<2, RW, EPI, RMS, kTail>, RW);
+        else if (a.K <= 2048)
+            launch(gemv_kernel<4, RW, EPI, RMS, kTail>, RW);
+        else if (a.K <= 4096)
+            launch(gemv_kernel<8, RW, EPI, RMS, kTail>, RW);
         else
-            grid = (a.N + RW - 1) / RW;
-        hipLaunchKernelGGL((gemv_kernel<4, RW, EPI, RMS>), dim3(grid), dim3(kWave), 0, s, a);
-    } else if (xa && a.K == 5632 && EPI != kEpiQKV && EPI != kEpiSwiglu) {
-        constexpr int RW = 2;
-        hipLaunchKernelGGL((gemv_kernel<11, RW, EPI, RMS>), dim3((a.N + RW - 1) / RW),
-                           dim3(kWave), 0, s, a);
+            launch(gemv_kernel<8, RW, EPI, RMS, kSlabs>, RW);
     } else {
         hipLaunchKernelGGL((gemv_generic_kernel<EPI, RMS>), dim3(units), dim3(kWave), 0, s, a);
     }
