@@ -96,6 +96,30 @@ int decode_attention_act(const void* q, const kvhp_kv_view* k_view, const kvhp_k
                          int num_kv_heads, int head_dim, int max_seq_len, void* workspace,
                          size_t workspace_bytes, int act_tiles, hipStream_t s);
 
+// gemm.hip: the prompt's projections, C[M][N] = A[M][K] W[N][K]^T with the
+// neighbouring row-wise work in the epilogue.  All tensors 16-byte aligned.
+// Shapes gemm_fits takes; SwiGLU wants F % 32 == 0 (N = 2F), q/k/v head_dim % 64 == 0.
+bool gemm_fits(int64_t M, int64_t N, int64_t K);
+// out += A W^T (fp16 residual stream); with a workspace of
+// gemm_residual_workspace bytes, few rows split K over more CUs
+size_t gemm_residual_workspace(int M, int N, int K);
+constexpr size_t kGemmWorkspace = size_t(4) << 20;   // enough for any shape
+int gemm_residual(const void* A, const void* W, void* out, int M, int N, int K, void* ws,
+                  size_t ws_bytes, hipStream_t s);
+// out[M][N] fp32
+int gemm_f32(const void* A, const void* W, float* out, int M, int N, int K, hipStream_t s);
+// out[M][F] = silu(gate) up of W_gate_up [gate; up] (both rounded to fp16 first)
+int gemm_swiglu(const void* A, const void* W_gate_up, void* out, int M, int F, int K,
+                hipStream_t s);
+// the fused q/k/v projection split into q, k, v with RoPE on q and k: row m
+// rotated by rope[m][D/2] (cos, sin), the products rounded to fp16 first
+int gemm_qkv(const void* A, const void* W_qkv, const float2* rope, void* q, void* k, void* v,
+             int M, int num_q_heads, int num_kv_heads, int head_dim, int K, hipStream_t s);
+// model_ops.hip: rope[m][D/2] = (cos, sin) of row m at position start + m, or at
+// positions[m] (device; negative: 0) when given.
+int rope_table(float2* rope, int64_t rows, int head_dim, int start, const int32_t* positions,
+               float theta, hipStream_t s);
+
 #define KVHP_REQUIRE(cond, code, ...)          \
     do {                                       \
         if (!(cond)) return ::kvhp::fail(code, __VA_ARGS__); \

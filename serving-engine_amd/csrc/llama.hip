@@ -22,10 +22,12 @@
 // K/V at its write position and attends over its seq_len keys; B sequences
 // go through each projection as one B-row GEMM.
 //
-// Prefill projections are library GEMMs (rocBLAS, fp16 in, fp32 compute,
-// fp16 out; the o and down projections accumulate into the residual stream
-// with beta = 1); attention is the flash prefill kernel, which also writes
-// the prompt's K/V pages.  Decode uses the fused GEMV kernels of
+// Prefill projections run on the MFMA kernels of gemm.hip, which add the
+// residual, apply SwiGLU, or split and rotate q/k/v as they store; dimensions
+// those do not take (K not a multiple of 64, odd head sizes) run on library
+// GEMMs (rocBLAS, fp16 in, fp32 compute, fp16 out) with separate launches.
+// Attention is the flash prefill kernel, which also writes the prompt's K/V
+// pages.  Decode uses the fused GEMV kernels of
 // model_ops.hip and the split-K decode attention of decode.hip.
 //
 // Synthetic weights: every matrix N(0, 0.02) in fp16 from the seeded
@@ -73,7 +75,7 @@ struct Model {
     std::vector<Layer> layers;
     f16* pool = nullptr;       // [L][2][Hkv][P][16][D], layer pools point into it
     int32_t* bt = nullptr;     // [P] identity page order
-    // prefill activations, sized for max_ctx rows
+    // prefill activations, sized for max_ctx rows (qkv and gu: library GEMMs only)
     f16 *hidden = nullptr, *norm = nullptr, *qkv = nullptr, *q = nullptr, *k = nullptr,
         *v = nullptr, *attn = nullptr, *gu = nullptr, *act = nullptr;
     // decode activations
@@ -95,6 +97,11 @@ struct Model {
     size_t part_rows_bytes = 0;
     int prompt_len = 0;
     bool rows_ok = false;      // batched projections fit the skinny-GEMM kernels
+    bool gemm_ok = false;      // prompt projections fit the kernels of gemm.hip
+    bool head_ok = false;      // so does the LM head of a large batch
+    float2* rope = nullptr;    // [max_ctx][D/2]: rotations of the rows of a forward
+    void* gemm_ws = nullptr;   // K-split partials of the residual projections
+    size_t gemm_ws_bytes = 0;
     f16* lm_head_t = nullptr;  // LM head tiled for the batched kernels
     bool tiled = false;        // the tiled copies hold the current weights
     // batched-step activations (2..32 rows), row-tiled (act_tiled_index):
@@ -182,6 +189,14 @@ int blas_check(rocblas_status st, const char* what) {
     return KVHP_OK;
 }
 
+// The library's handle, created with the model unless gemm.hip's kernels take all
+// of its shapes (an unaligned logits buffer creates it late).
+int need_blas(Model& m, hipStream_t s) {
+    if (m.blas) return KVHP_OK;
+    KVHP_TRY(blas_check(rocblas_create_handle(&m.blas), "rocblas_create_handle"));
+    return blas_check(rocblas_set_stream(m.blas, s), "rocblas_set_stream");
+}
+
 // C[M][N] (+)= A[M][K] W[N][K]^T, row-major, fp16 in/out, fp32 compute.
 int linear(Model& m, const f16* A, const f16* W, f16* C, int M, int N, int K, bool accumulate) {
     const float alpha = 1.f, beta = accumulate ? 1.f : 0.f;
@@ -248,13 +263,57 @@ kvhp_kv_view own_view(const Model& m, int l, int is_v) {
     return v;
 }
 
-// rocBLAS follows `s` for the lifetime of this object, then the model's
-// stream again.
+// rocBLAS (where the model uses it) follows `s` for the lifetime of this object,
+// then the model's stream again.
 struct BlasOn {
     Model& m;
-    BlasOn(Model& mm, hipStream_t s) : m(mm) { (void)rocblas_set_stream(m.blas, s); }
-    ~BlasOn() { (void)rocblas_set_stream(m.blas, m.stream); }
+    BlasOn(Model& mm, hipStream_t s) : m(mm) {
+        if (m.blas) (void)rocblas_set_stream(m.blas, s);
+    }
+    ~BlasOn() {
+        if (m.blas) (void)rocblas_set_stream(m.blas, m.stream);
+    }
 };
+
+// The projections of n rows.  On gemm.hip's kernels: QKV with the split and the
+// rotations of m.rope (filled once per forward), SwiGLU in the gate/up product.
+// Else a library GEMM and the row-wise kernel; row r at position start + r, or
+// at positions[r].
+int project_qkv(Model& m, const Layer& L, int n, int start, const int32_t* positions, void* s) {
+    const kvhp_llama_config& c = m.c;
+    const int H = c.hidden_size, D = c.head_dim, Hq = c.num_q_heads, Hkv = c.num_kv_heads;
+    if (m.gemm_ok)
+        return gemm_qkv(m.norm, L.w_qkv, m.rope, m.q, m.k, m.v, n, Hq, Hkv, D, H,
+                        static_cast<hipStream_t>(s));
+    KVHP_TRY(linear(m, m.norm, L.w_qkv, m.qkv, n, (Hq + 2 * Hkv) * D, H, false));
+    if (positions)
+        return kvhp_split_qkv_rope_rows(m.qkv, n, Hq, Hkv, D, positions, c.rope_theta, m.q, m.k,
+                                        m.v, s);
+    return kvhp_split_qkv_rope(m.qkv, n, Hq, Hkv, D, start, c.rope_theta, m.q, m.k, m.v, s);
+}
+
+int project_residual(Model& m, const f16* x, const f16* W, int n, int K, void* s) {
+    const int H = m.c.hidden_size;
+    if (m.gemm_ok)
+        return gemm_residual(x, W, m.hidden, n, H, K, m.gemm_ws, m.gemm_ws_bytes,
+                             static_cast<hipStream_t>(s));
+    return linear(m, x, W, m.hidden, n, H, K, true);
+}
+
+int project_swiglu(Model& m, const Layer& L, int n, void* s) {
+    const int H = m.c.hidden_size, F = m.c.ffn_size;
+    if (m.gemm_ok)
+        return gemm_swiglu(m.norm, L.w_gate_up, m.act, n, F, H, static_cast<hipStream_t>(s));
+    KVHP_TRY(linear(m, m.norm, L.w_gate_up, m.gu, n, 2 * F, H, false));
+    return kvhp_swiglu_rows(m.gu, m.act, n, F, s);
+}
+
+// The rotations of n rows, once per forward.
+int forward_rope(Model& m, int n, int start, const int32_t* positions, void* s) {
+    if (!m.gemm_ok) return KVHP_OK;
+    return rope_table(m.rope, n, m.c.head_dim, start, positions, m.c.rope_theta,
+                      static_cast<hipStream_t>(s));
+}
 
 // Prompt forward of m.tokens[0, n) (one sequence): final hidden rows in
 // m.hidden, the K/V of every position written through pg.bt (ids -1, pages
@@ -262,21 +321,20 @@ struct BlasOn {
 int prefill_layers(Model& m, int n, const Pages& pg, void* s) {
     const kvhp_llama_config& c = m.c;
     const int H = c.hidden_size, D = c.head_dim, Hq = c.num_q_heads, Hkv = c.num_kv_heads;
-    const int F = c.ffn_size, NQKV = (Hq + 2 * Hkv) * D;
+    const int F = c.ffn_size;
+    KVHP_TRY(forward_rope(m, n, 0, nullptr, s));
     KVHP_TRY(kvhp_embedding(m.tokens, m.embed, m.hidden, n, H, c.vocab_size, s));
     for (int l = 0; l < c.num_layers; ++l) {
         const Layer& L = m.layers[l];
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.attn_norm, m.norm, n, H, c.rms_eps, s));
-        KVHP_TRY(linear(m, m.norm, L.w_qkv, m.qkv, n, NQKV, H, false));
-        KVHP_TRY(kvhp_split_qkv_rope(m.qkv, n, Hq, Hkv, D, 0, c.rope_theta, m.q, m.k, m.v, s));
+        KVHP_TRY(project_qkv(m, L, n, 0, nullptr, s));
         KVHP_TRY(kvhp_flash_prefill_paged(m.q, m.k, m.v, m.attn, n, Hq, Hkv, D, 1,
                                           layer_pool(m, pg, l, 0), layer_pool(m, pg, l, 1), pg.bt,
                                           pg.max_pages, pg.num_pages, s));
-        KVHP_TRY(linear(m, m.attn, L.w_o, m.hidden, n, H, Hq * D, true));
+        KVHP_TRY(project_residual(m, m.attn, L.w_o, n, Hq * D, s));
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.ffn_norm, m.norm, n, H, c.rms_eps, s));
-        KVHP_TRY(linear(m, m.norm, L.w_gate_up, m.gu, n, 2 * F, H, false));
-        KVHP_TRY(kvhp_swiglu_rows(m.gu, m.act, n, F, s));
-        KVHP_TRY(linear(m, m.act, L.w_down, m.hidden, n, H, F, true));
+        KVHP_TRY(project_swiglu(m, L, n, s));
+        KVHP_TRY(project_residual(m, m.act, L.w_down, n, F, s));
     }
     return KVHP_OK;
 }
@@ -334,7 +392,7 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
                           hipStream_t s) {
     const kvhp_llama_config& c = m.c;
     const int H = c.hidden_size, D = c.head_dim, Hq = c.num_q_heads, Hkv = c.num_kv_heads;
-    const int F = c.ffn_size, NQKV = (Hq + 2 * Hkv) * D;
+    const int F = c.ffn_size;
     const int S = n - first;
     SuffixRows sr{};
     KVHP_TRY(suffix_rows(m, pg, write_bt, first, S, s, sr));
@@ -344,23 +402,22 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
     size_t ws_bytes = 0;
     KVHP_TRY(rows_workspace(m, S, n, s, &ws, &ws_bytes));
     const Pages rows_pg{pg.base, pg.num_pages, sr.tables, pg.max_pages};
+    KVHP_TRY(forward_rope(m, S, first, nullptr, s));
     KVHP_TRY(kvhp_embedding(m.tokens + first, m.embed, m.hidden, S, H, c.vocab_size, s));
     for (int l = 0; l < c.num_layers; ++l) {
         const Layer& L = m.layers[l];
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.attn_norm, m.norm, S, H, c.rms_eps, s));
-        KVHP_TRY(linear(m, m.norm, L.w_qkv, m.qkv, S, NQKV, H, false));
-        KVHP_TRY(kvhp_split_qkv_rope(m.qkv, S, Hq, Hkv, D, first, c.rope_theta, m.q, m.k, m.v, s));
+        KVHP_TRY(project_qkv(m, L, S, first, nullptr, s));
         KVHP_TRY(kvhp_paged_append_kv(m.k, m.v, layer_pool(m, pg, l, 0), layer_pool(m, pg, l, 1),
                                       write_bt, pg.max_pages, start, 1, S, Hkv, D, pg.num_pages,
                                       s));
         const kvhp_kv_view kv = pages_view(m, rows_pg, l, 0), vv = pages_view(m, rows_pg, l, 1);
         KVHP_TRY(kvhp_decode_attention(m.q, &kv, &vv, lens, m.attn, S, Hq, Hkv, D, n, 0, ws,
                                        ws_bytes, s));
-        KVHP_TRY(linear(m, m.attn, L.w_o, m.hidden, S, H, Hq * D, true));
+        KVHP_TRY(project_residual(m, m.attn, L.w_o, S, Hq * D, s));
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.ffn_norm, m.norm, S, H, c.rms_eps, s));
-        KVHP_TRY(linear(m, m.norm, L.w_gate_up, m.gu, S, 2 * F, H, false));
-        KVHP_TRY(kvhp_swiglu_rows(m.gu, m.act, S, F, s));
-        KVHP_TRY(linear(m, m.act, L.w_down, m.hidden, S, H, F, true));
+        KVHP_TRY(project_swiglu(m, L, S, s));
+        KVHP_TRY(project_residual(m, m.act, L.w_down, S, F, s));
     }
     return KVHP_OK;
 }
@@ -421,7 +478,7 @@ int decode_rows(Model& m, const int32_t* tokens, int B, const Pages& pg,
     const int32_t* wbt = write_bt ? write_bt : pg.bt;
     const kvhp_llama_config& c = m.c;
     const int H = c.hidden_size, D = c.head_dim, Hq = c.num_q_heads, Hkv = c.num_kv_heads;
-    const int F = c.ffn_size, NQKV = (Hq + 2 * Hkv) * D;
+    const int F = c.ffn_size;
     void* ws = nullptr;
     size_t ws_bytes = 0;
     KVHP_TRY(rows_workspace(m, B, max_seq_len, static_cast<hipStream_t>(s), &ws, &ws_bytes));
@@ -489,23 +546,27 @@ int decode_rows(Model& m, const int32_t* tokens, int B, const Pages& pg,
                                   logits, c.vocab_size, H, B, nt, hs));
         return kvhp_argmax_rows(logits, B, c.vocab_size, next, s);
     }
+    KVHP_TRY(forward_rope(m, B, 0, positions, s));
     for (int l = 0; l < c.num_layers; ++l) {
         const Layer& L = m.layers[l];
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.attn_norm, m.norm, B, H, c.rms_eps, s));
-        KVHP_TRY(linear(m, m.norm, L.w_qkv, m.qkv, B, NQKV, H, false));
-        KVHP_TRY(kvhp_split_qkv_rope_rows(m.qkv, B, Hq, Hkv, D, positions, c.rope_theta, m.q, m.k,
-                                          m.v, s));
+        KVHP_TRY(project_qkv(m, L, B, 0, positions, s));
         const kvhp_kv_view kv = pages_view(m, pg, l, 0), vv = pages_view(m, pg, l, 1);
         KVHP_TRY(kvhp_paged_append_decode(m.q, m.k, m.v, &kv, &vv, positions, seq_lens, m.attn, B,
                                           Hq, Hkv, D, max_seq_len, 0, ws, ws_bytes, s));
-        KVHP_TRY(linear(m, m.attn, L.w_o, m.hidden, B, H, Hq * D, true));
+        KVHP_TRY(project_residual(m, m.attn, L.w_o, B, Hq * D, s));
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.ffn_norm, m.norm, B, H, c.rms_eps, s));
-        KVHP_TRY(linear(m, m.norm, L.w_gate_up, m.gu, B, 2 * F, H, false));
-        KVHP_TRY(kvhp_swiglu_rows(m.gu, m.act, B, F, s));
-        KVHP_TRY(linear(m, m.act, L.w_down, m.hidden, B, H, F, true));
+        KVHP_TRY(project_swiglu(m, L, B, s));
+        KVHP_TRY(project_residual(m, m.act, L.w_down, B, F, s));
     }
     KVHP_TRY(kvhp_rmsnorm(m.hidden, m.final_norm, m.norm, B, H, c.rms_eps, s));
-    KVHP_TRY(linear_f32(m, m.norm, m.lm_head, logits, B, c.vocab_size, H));
+    if (m.head_ok && aligned16(logits))
+        KVHP_TRY(gemm_f32(m.norm, m.lm_head, logits, B, c.vocab_size, H,
+                          static_cast<hipStream_t>(s)));
+    else {
+        KVHP_TRY(need_blas(m, static_cast<hipStream_t>(s)));
+        KVHP_TRY(linear_f32(m, m.norm, m.lm_head, logits, B, c.vocab_size, H));
+    }
     return kvhp_argmax_rows(logits, B, c.vocab_size, next, s);
 }
 
@@ -559,12 +620,17 @@ extern "C" int kvhp_llama_create(const kvhp_llama_config* cfg, uint64_t seed, in
     m->max_ctx = max_ctx;
     m->P = (max_ctx + kPage - 1) / kPage;
     KVHP_HIP(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "hipStreamCreate");
-    KVHP_TRY(blas_check(rocblas_create_handle(&m->blas), "rocblas_create_handle"));
-    KVHP_TRY(blas_check(rocblas_set_stream(m->blas, m->stream), "rocblas_set_stream"));
-
     const int H = c.hidden_size, D = c.head_dim, Hq = c.num_q_heads, Hkv = c.num_kv_heads;
     const int F = c.ffn_size, V = c.vocab_size, S = max_ctx;
     const int NQKV = (Hq + 2 * Hkv) * D;
+    // every prompt projection on gemm.hip's kernels, or all on the library
+    m->gemm_ok = D % 64 == 0 && F % 64 == 0 && gemm_fits(S, NQKV, H) &&
+                 gemm_fits(S, H, Hq * D) && gemm_fits(S, 2 * (int64_t)F, H) && gemm_fits(S, H, F);
+    m->head_ok = gemm_fits(S, V, H);
+    if (!m->gemm_ok || !m->head_ok) {
+        KVHP_TRY(blas_check(rocblas_create_handle(&m->blas), "rocblas_create_handle"));
+        KVHP_TRY(blas_check(rocblas_set_stream(m->blas, m->stream), "rocblas_set_stream"));
+    }
     void* s = m->stream;
     uint64_t tensor_id = 0;
     auto randn = [&](f16** p, size_t n) {
@@ -608,12 +674,18 @@ extern "C" int kvhp_llama_create(const kvhp_llama_config* cfg, uint64_t seed, in
     }
     KVHP_TRY(alloc_n(*m, (size_t)S * H, &m->hidden));
     KVHP_TRY(alloc_n(*m, (size_t)S * H, &m->norm));
-    KVHP_TRY(alloc_n(*m, (size_t)S * NQKV, &m->qkv));
+    if (m->gemm_ok) {
+        KVHP_TRY(alloc_n(*m, (size_t)S * (D / 2), &m->rope));
+        m->gemm_ws_bytes = kGemmWorkspace;
+        KVHP_TRY(alloc(*m, m->gemm_ws_bytes, &m->gemm_ws));
+    } else {
+        KVHP_TRY(alloc_n(*m, (size_t)S * NQKV, &m->qkv));
+        KVHP_TRY(alloc_n(*m, (size_t)S * 2 * F, &m->gu));
+    }
     KVHP_TRY(alloc_n(*m, (size_t)S * Hq * D, &m->q));
     KVHP_TRY(alloc_n(*m, (size_t)S * Hkv * D, &m->k));
     KVHP_TRY(alloc_n(*m, (size_t)S * Hkv * D, &m->v));
     KVHP_TRY(alloc_n(*m, (size_t)S * Hq * D, &m->attn));
-    KVHP_TRY(alloc_n(*m, (size_t)S * 2 * F, &m->gu));
     KVHP_TRY(alloc_n(*m, (size_t)S * F, &m->act));
     KVHP_TRY(alloc_n(*m, H, &m->x));
     KVHP_TRY(alloc_n(*m, (size_t)Hq * D, &m->q1));

@@ -1232,6 +1232,20 @@ __global__ void split_qkv_rope_kernel(const f16* qkv, int64_t S, int Hq, int Hkv
     }
 }
 
+// (cos, sin) of every row and dimension pair: one prompt's (or batched step's)
+// rotations, computed once for all layers.
+__global__ void __launch_bounds__(256)
+rope_table_kernel(float2* rope, int64_t n, int half, int D, int start, const int32_t* positions,
+                  float theta) {
+    const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (t >= n) return;
+    const int64_t m = t / half;
+    const int pos = positions ? max(positions[m], 0) : static_cast<int>(start + m);
+    float2 r;
+    rope_cs(pos, static_cast<int>(t % half), D, theta, r.x, r.y);
+    rope[t] = r;
+}
+
 // The same for D % 16 == 0 and 16-byte aligned tensors.  A workgroup takes TB
 // tokens and computes each token's D/2 rotations once, into LDS, for all of
 // its heads (one powf, cosf and sinf per pair and head cost more than the
@@ -2097,6 +2111,16 @@ extern "C" int kvhp_argmax_rows(const float* logits, int64_t rows, int64_t n, in
 }
 
 namespace kvhp {
+int rope_table(float2* rope, int64_t rows, int head_dim, int start, const int32_t* positions,
+               float theta, hipStream_t s) {
+    const int half = head_dim / 2;
+    const int64_t n = rows * half;
+    if (n <= 0) return KVHP_OK;
+    hipLaunchKernelGGL(rope_table_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256),
+                       0, s, rope, n, half, head_dim, start, positions, theta);
+    return check_launch("rope_table");
+}
+
 int argmax_embed(const float* logits, int64_t n, int32_t* token, int32_t* seq_len, int32_t* log,
                  int32_t* log_count, const void* embed, int64_t hidden, void* x, hipStream_t s) {
     KVHP_REQUIRE(logits && token && embed && x && n > 0 && n < (int64_t)1 << 31 && hidden > 0,
