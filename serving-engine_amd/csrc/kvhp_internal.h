@@ -96,6 +96,15 @@ int decode_attention_act(const void* q, const kvhp_kv_view* k_view, const kvhp_k
                          int num_kv_heads, int head_dim, int max_seq_len, void* workspace,
                          size_t workspace_bytes, int act_tiles, hipStream_t s);
 
+// prefill.hip: causal attention of a prompt's last `rows` positions (first ..)
+// over keys read from the pages of one block-table row, which hold all
+// first + rows of them; q, out [rows][Hq][D] 16-byte aligned.  Few rows split
+// the keys: the workspace holds the fp32 partials.
+bool prefill_cached_fits(int rows, int first, int hq, int hkv, int d);
+size_t prefill_cached_workspace(int rows, int first, int hq, int hkv, int d);
+int prefill_cached(const void* q, const void* pool_k, const void* pool_v, const int32_t* bt,
+                   int max_pages, int num_pages, void* out, int rows, int first, int hq,
+                   int hkv, int d, void* ws, size_t ws_bytes, hipStream_t s);
 // gemm.hip: the prompt's projections, C[M][N] = A[M][K] W[N][K]^T with the
 // neighbouring row-wise work in the epilogue.  All tensors 16-byte aligned.
 // Shapes gemm_fits takes; SwiGLU wants F % 32 == 0 (N = 2F), q/k/v head_dim % 64 == 0.

@@ -169,10 +169,13 @@ int regrow(Model& m, T** p, size_t* cap, size_t n, hipStream_t s, const char* wh
 // Decode-attention workspace for B sequences of up to max_seq_len keys,
 // owned by the model (not the library's per-device buffer), so that models
 // on different streams never share split partials.
-int rows_workspace(Model& m, int B, int max_seq_len, hipStream_t s, void** ws, size_t* bytes) {
+// With `bytes_needed` that size instead (the cached-prefix attention's partials).
+int rows_workspace(Model& m, int B, int max_seq_len, hipStream_t s, void** ws, size_t* bytes,
+                   size_t bytes_needed = 0) {
     const kvhp_llama_config& c = m.c;
-    const size_t need = kvhp_decode_workspace_bytes(B, c.num_q_heads, c.num_kv_heads, c.head_dim,
-                                                    max_seq_len, 0);
+    const size_t need = bytes_needed ? bytes_needed
+                                     : kvhp_decode_workspace_bytes(B, c.num_q_heads, c.num_kv_heads,
+                                                                   c.head_dim, max_seq_len, 0);
     if (need > m.ws_rows_bytes) {
         char* p = static_cast<char*>(m.ws_rows);
         KVHP_TRY(regrow(m, &p, &m.ws_rows_bytes, need, s, "decode-attention workspace"));
@@ -386,7 +389,8 @@ int suffix_rows(Model& m, const Pages& pg, const int32_t* write_bt, int first, i
 // model (m.tokens holds all n ids).  Their K/V are appended through
 // write_bt (the block-table row, or it with shared pages set to -1), and
 // query row r attends over keys
-// [0, first + r + 1) from the pages -- the cached prefix included -- as one
+// [0, first + r + 1) from the pages -- the cached prefix included -- by the
+// flash prefill kernel on pages, or for shapes it does not take as one
 // row of a batched decode-attention call.  Final hidden rows in m.hidden.
 int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int32_t* write_bt,
                           hipStream_t s) {
@@ -400,7 +404,9 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
     int32_t* start = sr.start;
     void* ws = nullptr;
     size_t ws_bytes = 0;
-    KVHP_TRY(rows_workspace(m, S, n, s, &ws, &ws_bytes));
+    const bool flash = prefill_cached_fits(S, first, Hq, Hkv, D) && aligned16(pg.base);
+    KVHP_TRY(rows_workspace(m, S, n, s, &ws, &ws_bytes,
+                            flash ? prefill_cached_workspace(S, first, Hq, Hkv, D) : 0));
     const Pages rows_pg{pg.base, pg.num_pages, sr.tables, pg.max_pages};
     KVHP_TRY(forward_rope(m, S, first, nullptr, s));
     KVHP_TRY(kvhp_embedding(m.tokens + first, m.embed, m.hidden, S, H, c.vocab_size, s));
@@ -411,9 +417,15 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
         KVHP_TRY(kvhp_paged_append_kv(m.k, m.v, layer_pool(m, pg, l, 0), layer_pool(m, pg, l, 1),
                                       write_bt, pg.max_pages, start, 1, S, Hkv, D, pg.num_pages,
                                       s));
-        const kvhp_kv_view kv = pages_view(m, rows_pg, l, 0), vv = pages_view(m, rows_pg, l, 1);
-        KVHP_TRY(kvhp_decode_attention(m.q, &kv, &vv, lens, m.attn, S, Hq, Hkv, D, n, 0, ws,
-                                       ws_bytes, s));
+        if (flash) {
+            KVHP_TRY(prefill_cached(m.q, layer_pool(m, pg, l, 0), layer_pool(m, pg, l, 1), pg.bt,
+                                    pg.max_pages, pg.num_pages, m.attn, S, first, Hq, Hkv, D, ws,
+                                    ws_bytes, s));
+        } else {
+            const kvhp_kv_view kv = pages_view(m, rows_pg, l, 0), vv = pages_view(m, rows_pg, l, 1);
+            KVHP_TRY(kvhp_decode_attention(m.q, &kv, &vv, lens, m.attn, S, Hq, Hkv, D, n, 0, ws,
+                                           ws_bytes, s));
+        }
         KVHP_TRY(project_residual(m, m.attn, L.w_o, S, Hq * D, s));
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.ffn_norm, m.norm, S, H, c.rms_eps, s));
         KVHP_TRY(project_swiglu(m, L, S, s));

@@ -38,6 +38,10 @@
 // alternate an MFMA step (S^T of tile j, O^T of tile j-1, operand reads
 // scheduled ahead, at wave priority 1) and a softmax step one phase apart.
 //
+// With 5..8 query heads per KV head the same split runs with a KV head's query
+// heads on two workgroups.  A prompt's last positions behind a cached prefix
+// run on the same kernel with the keys read from their pages.
+//
 // With a page pool, each workgroup also writes the K/V rows of its own query
 // block into the pages after its outputs (every key row is written exactly
 // once, bit-exact).
@@ -46,6 +50,7 @@
 // flops (the two causal contractions).
 #include "kvhp_internal.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace kvhp {
@@ -70,6 +75,16 @@ struct PrefillArgs {
     int n_qblk;
     int paired;             // 1: query blocks i and n-1-i share a workgroup (two passes)
     float scale_log2;
+    int HG, nsub;           // SUB: query heads per workgroup, workgroups per KV head
+    int fold;               // unpaired: the longer half of the blocks longest first, then the
+                            // shorter half shortest first (two workgroups per CU)
+    // CACHED: the q rows sit at positions first .. first + S - 1 and all keys are
+    // read from the pages (k, v: the pools; bt, max_pages, num_pages as above).
+    int first;
+    int tiles_per_split;    // key tiles of a split (blockIdx.z)
+    int nsplit;
+    float* ws_o;            // [S * Hq][nsplit][D], nsplit > 1
+    float* ws_ml;           // [S * Hq][nsplit][2]  (max in log2 units, sum)
 };
 
 typedef short short4v __attribute__((ext_vector_type(4)));
@@ -159,7 +174,19 @@ __device__ __forceinline__ float halves_sum(float x) {
 //                   16t + 4h + e for e < 4 and 16t + 8 + 4h + e - 4 above.
 // Per 64-key tile a wave does 32 MFMAs (1 MFLOP) for 32 KB of LDS reads,
 // twice the work per LDS byte of 16x16 tiles.
-template <int D, int KG>
+//
+// SUB: a KV head's query heads are cut into nsub groups of at most HG, a
+// workgroup each (G = 5..8 at KG = 2).
+//
+// CACHED: attention of a prompt's last S positions over keys in pages, the
+// cached prefix included.  A tile's four pages are loaded through their ids,
+// which sit in LDS from the start (a load from the block table inside the loop
+// would wait for every DMA in flight).  Few query rows leave CUs idle, so the
+// keys may be cut into nsplit ranges; a row whose keys reach past the first
+// stores its partial (m, l, O) for prefill_merge_kernel.
+constexpr int kMaxTablePages = 4096;   // page ids of a split in LDS (65536 keys)
+
+template <int D, int KG, bool SUB, bool CACHED>
 __global__ void __launch_bounds__(8 * kWave)
 prefill_mfma_kernel(const PrefillArgs a) {
     constexpr int WAVES = 8;
@@ -172,7 +199,10 @@ prefill_mfma_kernel(const PrefillArgs a) {
     constexpr int IPW = kBN / RPI / WAVES;  // DMA instructions per wave per matrix
     constexpr int LPT = 2 * IPW;        // DMA loads per wave per tile (K + V)
     constexpr int TB = kBN * D;         // halfs per tile matrix
-    constexpr int KSW = CPR - 1;        // K swizzle: c ^ (r & KSW)
+    // K swizzle: 16 consecutive rows of one chunk cover the 16 slots of a
+    // 256-byte bank line (D = 64: two rows a line; c ^ (r & 7) there read rows r
+    // and r + 8 from the same banks, half of the LDS cycles).
+    auto kswz = [](int r) { return CPR == 16 ? r & 15 : r >> 1 & 7; };
     // V swizzle: the transposing reads of one half-wave touch 4 consecutive
     // rows x 4 chunks; these land on distinct 16-byte bank groups of the
     // 256-byte bank line.
@@ -180,6 +210,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
 
     constexpr int NSTAGE = 4;
     __shared__ __attribute__((aligned(16))) f16 ring[NSTAGE * 2 * TB];
+    __shared__ int32_t ptab[CACHED ? kMaxTablePages : 1];
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS bases in SGPRs
@@ -189,18 +220,26 @@ prefill_mfma_kernel(const PrefillArgs a) {
     const int j16 = lane & 15;      // lane within its 16-lane block
     const int blk2 = (lane >> 4) & 1;
 
-    const int kvh = blockIdx.x % a.Hkv;
-    const int pair = blockIdx.x / a.Hkv;   // pair index (paired) or block rank, longest first
+    const int hw = SUB ? a.Hkv * a.nsub : a.Hkv;   // workgroups per block or pair
+    const int kvh = SUB ? blockIdx.x % hw / a.nsub : blockIdx.x % a.Hkv;
+    const int sub = SUB ? blockIdx.x % hw % a.nsub : 0;
+    const int pair = blockIdx.x / hw;   // pair index (paired) or block rank, longest first
     const int b = blockIdx.y;
     const int S = a.S;
-    const int G = a.G;
+    const int G = SUB ? min(a.HG, a.G - sub * a.HG) : a.G;   // this workgroup's query heads
+    const int head0 = kvh * a.G + sub * a.HG;                // and the first of them
+    const int first = CACHED ? a.first : 0;
+    const int n_keys = first + S;
+    const int t_lo = CACHED ? static_cast<int>(blockIdx.z) * a.tiles_per_split : 0;
     const int RB = a.RB;
     const int BM = 32 * RB;
     const int nunits = G * RB;
     const int64_t qrs = (int64_t)a.Hq * D;     // q/out row stride
     const int64_t kvrs = (int64_t)a.Hkv * D;   // k/v row stride
-    const f16* kb = a.k + (int64_t)b * S * kvrs + (int64_t)kvh * D;
-    const f16* vb = a.v + (int64_t)b * S * kvrs + (int64_t)kvh * D;
+    const f16* kb = CACHED ? a.k + (int64_t)kvh * a.num_pages * kPage * D
+                           : a.k + (int64_t)b * S * kvrs + (int64_t)kvh * D;
+    const f16* vb = CACHED ? a.v + (int64_t)kvh * a.num_pages * kPage * D
+                           : a.v + (int64_t)b * S * kvrs + (int64_t)kvh * D;
 
     // DMA of tile tt into a stage: this wave's rows (wave*IPW + p)*RPI + lane/CPR.
     // Tiles past the last one re-load the last tile (an L2 hit): every path
@@ -210,13 +249,33 @@ prefill_mfma_kernel(const PrefillArgs a) {
 #pragma unroll
     for (int p = 0; p < IPW; ++p) {
         const int row = (wave * IPW + p) * RPI + lane / CPR;
-        const int ck = (lane % CPR) ^ (row & KSW);
+        const int ck = (lane % CPR) ^ kswz(row);
         const int cv = (lane % CPR) ^ vswz(row);
         dko[p] = static_cast<uint32_t>((row * kvrs + 8 * ck) * 2);
         dvo[p] = static_cast<uint32_t>((row * kvrs + 8 * cv) * 2);
     }
     int last_tile = 0;
+    // CACHED: this wave's 8 rows of a tile lie in page wave / 2 of its four.
+    const int last_pi = (n_keys - 1) >> 4, last_slot = (n_keys - 1) & 15;
+    int pid_next = 0;   // page id of the next issue, read one issue ahead
+    auto page_of = [&](int tt) { return min((t_lo + min(tt, last_tile)) * 4 + (wave >> 1), last_pi); };
     auto issue = [&](f16* stg, int tt) {
+        if constexpr (CACHED) {
+            // rows past the context's last token re-read its row (finite)
+            const int pu = (t_lo + min(tt, last_tile)) * 4 + (wave >> 1);
+            const int lim = pu >= last_pi ? last_slot : kPage - 1;
+            const int64_t page = (int64_t)__builtin_amdgcn_readfirstlane(pid_next) * (kPage * D);
+#pragma unroll
+            for (int p = 0; p < IPW; ++p) {
+                const int blk = wave * IPW + p;
+                const int row = blk * RPI + lane / CPR;
+                const uint32_t src = static_cast<uint32_t>(min(row & (kPage - 1), lim) * D * 2);
+                dma16s(kb + page, src + 16 * ((lane % CPR) ^ kswz(row)), stg + blk * RPI * D);
+                dma16s(vb + page, src + 16 * ((lane % CPR) ^ vswz(row)), stg + TB + blk * RPI * D);
+            }
+            pid_next = ptab[page_of(tt + 1) - t_lo * 4];
+            return;
+        }
         tt = min(tt, last_tile);
         const int key0 = tt * kBN;
         if (key0 + kBN <= S) {
@@ -235,7 +294,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
                 const int blk = wave * IPW + p;
                 const int row = blk * RPI + lane / CPR;
                 const int key = min(key0 + row, S - 1);
-                const int ck = (lane % CPR) ^ (row & KSW);
+                const int ck = (lane % CPR) ^ kswz(row);
                 const int cv = (lane % CPR) ^ vswz(row);
                 dma16(kb + (int64_t)key * kvrs + 8 * ck, stg + blk * RPI * D);
                 dma16(vb + (int64_t)key * kvrs + 8 * cv, stg + TB + blk * RPI * D);
@@ -251,7 +310,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
         const int r = 32 * kgrp_ + c32;
-        kro[c] = r * D + 8 * ((2 * c + h) ^ (r & KSW));
+        kro[c] = r * D + 8 * ((2 * c + h) ^ kswz(r));
     }
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
@@ -273,6 +332,8 @@ prefill_mfma_kernel(const PrefillArgs a) {
         } else {
             if (pass == 1) break;
             qblk = a.n_qblk - 1 - pair;   // one block per workgroup, longest first
+            if (D == 64 && KG == 2)
+                if (a.fold && pair >= (a.n_qblk + 1) / 2) qblk = pair - (a.n_qblk + 1) / 2;
         }
         const int q0 = qblk * BM;
 
@@ -281,7 +342,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
         const int u = wave % UPG;
         const int kgrp = wave / UPG;
         const bool uvalid = u < nunits;
-        const int qh = kvh * G + (uvalid ? u % G : 0);
+        const int qh = (SUB ? head0 : kvh * G) + (uvalid ? u % G : 0);
         const int r0 = q0 + 32 * (uvalid ? u / G : 0);
         const int row = r0 + c32;
         half8 qop[NC];
@@ -300,8 +361,22 @@ prefill_mfma_kernel(const PrefillArgs a) {
         const float lazy_thr = kLazyLog2 / a.scale_log2;   // in raw score units
 
         const int last_row = min(q0 + BM, S) - 1;
-        const int n_tiles = last_row / kBN + 1;
+        int n_tiles = (first + last_row) / kBN + 1;
+        if constexpr (CACHED) {
+            n_tiles = min(n_tiles - t_lo, a.tiles_per_split);
+            if (n_tiles <= 0) return;   // the block's keys end before this split
+        }
         last_tile = n_tiles - 1;
+        if constexpr (CACHED) {
+            // the split's page ids, clamped into the pool
+            const int np = min(n_tiles * 4, last_pi - t_lo * 4 + 1);
+            for (int i = tid; i < np; i += NTH) {
+                const int pid = t_lo * 4 + i < a.max_pages ? a.bt[t_lo * 4 + i] : 0;
+                ptab[i] = min(max(pid, 0), a.num_pages - 1);
+            }
+            __syncthreads();
+            pid_next = ptab[page_of(0) - t_lo * 4];
+        }
 
         wait_vmcnt<0>();  // q in registers before the ring: no compiler waits inside it
         ring_barrier();   // everyone is done with the previous pass's stages
@@ -386,17 +461,17 @@ prefill_mfma_kernel(const PrefillArgs a) {
             __builtin_amdgcn_s_setprio(0);
         };
         auto sstep = [&](int j) {
-            const int k0 = j * kBN;
-            const bool act = uvalid && k0 <= r0 + 31;
+            const int k0 = (t_lo + j) * kBN;
+            const bool act = uvalid && k0 <= first + r0 + 31;
             // ---- online softmax of query row `row`; P^T operands straight
             // from S^T.  Inactive units (invalid, or entirely above the
             // diagonal) see only -inf scores: alpha = 1 and p = 0 leave their
             // state as is.  The running max is kept on raw scores and the
             // scale folded into the exponent.
-            if (!act || k0 + kBN - 1 > r0) {
+            if (!act || k0 + kBN - 1 > first + r0) {
                 // element (kb2, i) holds key k0 + 32(kb2 + kgrp) + 4h +
                 // 8(i/4) + i%4; keys past min(row, S-1) are masked
-                const int lim = act ? min(row, S - 1) - (k0 + 32 * kgrp + 4 * h) : -1;
+                const int lim = act ? min(first + row, n_keys - 1) - (k0 + 32 * kgrp + 4 * h) : -1;
 #pragma unroll
                 for (int kb2 = 0; kb2 < NKB; ++kb2)
 #pragma unroll
@@ -479,7 +554,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
         //      of the pass's last tile come from its ring stage (still intact:
         //      the trailing re-loads go to the other stages), earlier rows
         //      (blocks longer than a tile) from memory.
-        if (a.pool_k) {
+        if (!CACHED && a.pool_k && (!SUB || sub == 0)) {
             const int lt0 = last_tile * kBN;
             const f16* Ks = ring + (last_tile % NSTAGE) * 2 * TB;
             const f16* Vs = Ks + TB;
@@ -494,7 +569,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
                 half8 kk, vv;
                 if (key >= lt0) {
                     const int r = key - lt0;
-                    kk = *reinterpret_cast<const half8*>(&Ks[r * D + 8 * (ch ^ (r & KSW))]);
+                    kk = *reinterpret_cast<const half8*>(&Ks[r * D + 8 * (ch ^ kswz(r))]);
                     vv = *reinterpret_cast<const half8*>(&Vs[r * D + 8 * (ch ^ vswz(r))]);
                 } else {
                     kk = load_half8(kb + (int64_t)key * kvrs + 8 * ch);
@@ -531,6 +606,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
                 const float mn = fmaxf(m_run, m1);
                 const float a0 = fast_exp2((m_run - mn) * a.scale_log2);
                 const float a1 = fast_exp2((m1 - mn) * a.scale_log2);
+                if constexpr (CACHED) m_run = mn;   // O and l are relative to it from here
                 l_part = l_part * a0 + l1 * a1;
 #pragma unroll
                 for (int db = 0; db < NDB; ++db)
@@ -548,7 +624,24 @@ prefill_mfma_kernel(const PrefillArgs a) {
         // ---- normalise and store: lane holds row `row`, dims 32db + 8q + 4h + e.
         {
             const float lt = halves_sum(l_part);
-            if (kgrp == 0 && uvalid && row < S) {
+            // a row whose keys reach past one split leaves its partial for the merge
+            const int per_split = CACHED ? a.tiles_per_split * kBN : 0;
+            if (CACHED && kgrp == 0 && uvalid && row < S && first + row >= per_split) {
+                // (splits past the row's keys are not read by the merge)
+                const int64_t prow = ((int64_t)row * a.Hq + qh) * a.nsplit + blockIdx.z;
+                float* po = a.ws_o + prow * D + 4 * h;
+#pragma unroll
+                for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4)
+                        *reinterpret_cast<floatx4*>(po + 32 * db + 8 * q4) =
+                            floatx4{o[db][4 * q4], o[db][4 * q4 + 1], o[db][4 * q4 + 2],
+                                    o[db][4 * q4 + 3]};
+                if (h == 0) {
+                    a.ws_ml[prow * 2] = m_run * a.scale_log2;
+                    a.ws_ml[prow * 2 + 1] = lt;
+                }
+            } else if (kgrp == 0 && uvalid && row < S && (!CACHED || blockIdx.z == 0)) {
                 const float inv = lt > 0.f ? 1.f / lt : 0.f;
                 f16* orow = a.out + ((int64_t)b * S + row) * qrs + (int64_t)qh * D + 4 * h;
 #pragma unroll
@@ -565,6 +658,55 @@ prefill_mfma_kernel(const PrefillArgs a) {
 
         wait_vmcnt<0>();   // page and output stores complete before the next ring starts
     }
+}
+
+// Log-sum-exp merge of the key splits' partials, 8 dims of one (row, head) a
+// thread; rows whose keys lie in the first split were written directly.  One
+// workgroup per (head, row) as decode's merges take 20 us more at 512 rows of
+// 32 heads.
+__global__ void __launch_bounds__(256)
+prefill_merge_kernel(const float* ws_o, const float* ws_ml, f16* out, int64_t threads, int Hq,
+                     int D, int first, int keys_per_split, int nsplit) {
+    const int64_t t = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (t >= threads) return;
+    const int cpr = D / 8, c = static_cast<int>(t % cpr);
+    const int64_t rh = t / cpr;
+    const int n = static_cast<int>((first + rh / Hq + keys_per_split) / keys_per_split);   // its splits
+    if (n <= 1) return;
+    const float* po = ws_o + rh * nsplit * D + 8 * c;
+    const float2* pml = reinterpret_cast<const float2*>(ws_ml) + rh * nsplit;
+    float M = -3.0e38f, L = 0.f;
+    floatx4 o0 = {0.f, 0.f, 0.f, 0.f}, o1 = o0;
+    constexpr int U = 4;   // splits in flight
+    for (int j0 = 0; j0 < n; j0 += U) {
+        float2 ml[U];
+        floatx4 x[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = min(j0 + u, n - 1);
+            ml[u] = pml[j];
+            x[u][0] = *reinterpret_cast<const floatx4*>(po + (int64_t)j * D);
+            x[u][1] = *reinterpret_cast<const floatx4*>(po + (int64_t)j * D + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j0 + u >= n) continue;
+            const float mn = fmaxf(M, ml[u].x);
+            const float al = fast_exp2(M - mn), be = fast_exp2(ml[u].x - mn);
+            o0 = o0 * al + x[u][0] * be;
+            o1 = o1 * al + x[u][1] * be;
+            L = fmaf(L, al, ml[u].y * be);
+            M = mn;
+        }
+    }
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    half8 h;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        h[e] = static_cast<f16>(o0[e] * inv);
+        h[4 + e] = static_cast<f16>(o1[e] * inv);
+    }
+    store_half8(out + rh * D + 8 * c, h);
 }
 
 // Any head_dim <= 256 / any alignment: one wave per (query head, row),
@@ -651,7 +793,7 @@ int prefill_impl(const void* q, const void* k, const void* v, void* out, int64_t
                      "flash_prefill_paged: %d pages per sequence cannot hold %lld tokens",
                      max_pages, (long long)seq_len);
     }
-    PrefillArgs a;
+    PrefillArgs a{};
     a.q = static_cast<const f16*>(q);
     a.k = static_cast<const f16*>(k);
     a.v = static_cast<const f16*>(v);
@@ -687,28 +829,127 @@ int prefill_impl(const void* q, const void* k, const void* v, void* out, int64_t
         const int64_t qblk1 = (seq_len + 32 * (8 / a.G) - 1) / (32 * (8 / a.G));
         const int64_t grid1 = (int64_t)hkv * ((qblk1 + 1) / 2) * batch;
         const bool split = grid1 <= kNumCUs / 2 || (grid1 > kNumCUs && grid1 <= kNumCUs * 3 / 2);
-        const int kg = ((a.G == 1 || a.G == 2 || a.G == 4) && split) ? 2 : 1;
-        a.RB = 8 / kg / a.G;
+        // G = 5..8 take the same split with the heads cut in two (SUB).  Us before
+        // and after at D = 64: 14/2 heads 3 x 777 21.6 / 16.9, 512 15.3 / 12.0,
+        // 2048 45.4 / 34.3, 4096 84.5 / 65.3; 32/4 heads 1024 24.3 / 17.5, 2048
+        // 41.8 / 31.8; at D = 128, 32/4 heads 2048 59.5 / 47.5, 6000 345 / 325;
+        // outside the rule (32/4 x 64 at 4096 and 8192) it is 2-4 % slower.
+        const bool sub = a.G > 4 && split;
+        const int kg = sub || ((a.G == 1 || a.G == 2 || a.G == 4) && split) ? 2 : 1;
+        a.nsub = sub ? 2 : 1;
+        a.HG = (a.G + a.nsub - 1) / a.nsub;
+        a.RB = sub ? 1 : 8 / kg / a.G;
         const int bm = 32 * a.RB;
         a.n_qblk = static_cast<int>((seq_len + bm - 1) / bm);
         // pair the causal blocks only when the pairs fill every CU
-        const int64_t pgrid = (int64_t)hkv * ((a.n_qblk + 1) / 2) * batch;
+        const int64_t pgrid = (int64_t)hkv * a.nsub * ((a.n_qblk + 1) / 2) * batch;
         a.paired = (pgrid >= kNumCUs) ? 1 : 0;
-        dim3 grid(hkv * (a.paired ? (a.n_qblk + 1) / 2 : a.n_qblk), batch);
+        // D = 64 at KG = 2 keeps two workgroups on a CU (64 KB LDS, 125 VGPRs):
+        // while every block is resident at once, a block each, the long half
+        // ahead of the short half in reverse, so that a CU's two add up alike
+        // (32/8 heads 2048 34.5 paired / 32.6, 32/4 heads 33.1 / 31.8).
+        if (d == 64 && kg == 2 && (int64_t)hkv * a.nsub * a.n_qblk * batch <= 2 * kNumCUs) {
+            a.paired = 0;
+            a.fold = 1;
+        }
+        dim3 grid(hkv * a.nsub * (a.paired ? (a.n_qblk + 1) / 2 : a.n_qblk), batch);
         const dim3 blk(8 * kWave);
-        if (d == 64 && kg == 2)
-            hipLaunchKernelGGL((prefill_mfma_kernel<64, 2>), grid, blk, 0, s, a);
-        else if (d == 64)
-            hipLaunchKernelGGL((prefill_mfma_kernel<64, 1>), grid, blk, 0, s, a);
-        else if (kg == 2)
-            hipLaunchKernelGGL((prefill_mfma_kernel<128, 2>), grid, blk, 0, s, a);
+        auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, 0, s, a); };
+        if (d == 64)
+            sub ? launch(prefill_mfma_kernel<64, 2, true, false>)
+                : kg == 2 ? launch(prefill_mfma_kernel<64, 2, false, false>)
+                          : launch(prefill_mfma_kernel<64, 1, false, false>);
         else
-            hipLaunchKernelGGL((prefill_mfma_kernel<128, 1>), grid, blk, 0, s, a);
+            sub ? launch(prefill_mfma_kernel<128, 2, true, false>)
+                : kg == 2 ? launch(prefill_mfma_kernel<128, 2, false, false>)
+                          : launch(prefill_mfma_kernel<128, 1, false, false>);
         return check_launch("flash_prefill");
     }
     dim3 grid(hq, static_cast<unsigned>(seq_len), batch);
     hipLaunchKernelGGL(prefill_generic_kernel, grid, dim3(kWave), 0, s, a, d);
     return check_launch("flash_prefill(generic)");
+}
+
+// The cached-prefix plan: query blocks of 32 rows (KG = 2), all of a block's
+// keys in one split when the blocks fill the CUs, else in ranges of at least 4
+// tiles so that about kNumCUs workgroups run.  Two layers with 512 new tokens
+// behind 1488 cached (32/4 heads of 64) in us, aiming at 128 / 256 / 512 / 1024
+// workgroups: 327 / 317 / 323 / 356 (489 as decode rows, which read the keys once
+// per query row).
+struct CachedPlan {
+    int nsub, HG, RB, n_qblk, nsplit, tiles;
+};
+
+static bool cached_plan(int rows, int first, int hq, int hkv, int d, CachedPlan& p) {
+    const int G = hq / hkv;
+    if ((d != 64 && d != 128) || G > 8 || G == 3) return false;
+    p.nsub = G > 4 ? 2 : 1;
+    p.HG = (G + p.nsub - 1) / p.nsub;
+    p.RB = G > 4 ? 1 : 4 / G;
+    p.n_qblk = (rows + 32 * p.RB - 1) / (32 * p.RB);
+    const int64_t wgs = (int64_t)hkv * p.nsub * p.n_qblk;
+    const int tiles = (first + rows + kBN - 1) / kBN;
+    int n = static_cast<int>(std::min<int64_t>(kNumCUs / std::max<int64_t>(wgs, 1), tiles / 4));
+    n = std::max(n, (tiles * 4 + kMaxTablePages - 1) / kMaxTablePages);   // page ids in LDS
+    n = std::max(n, 1);
+    p.tiles = (tiles + n - 1) / n;
+    p.nsplit = (tiles + p.tiles - 1) / p.tiles;
+    return p.nsplit <= 64;
+}
+
+size_t prefill_cached_workspace(int rows, int first, int hq, int hkv, int d) {
+    CachedPlan p;
+    if (!cached_plan(rows, first, hq, hkv, d, p) || p.nsplit == 1) return 0;
+    return sizeof(float) * (size_t)rows * hq * p.nsplit * (d + 2);
+}
+
+bool prefill_cached_fits(int rows, int first, int hq, int hkv, int d) {
+    CachedPlan p;
+    return cached_plan(rows, first, hq, hkv, d, p);
+}
+
+int prefill_cached(const void* q, const void* pool_k, const void* pool_v, const int32_t* bt,
+                   int max_pages, int num_pages, void* out, int rows, int first,
+                   int hq, int hkv, int d, void* ws, size_t ws_bytes, hipStream_t s) {
+    CachedPlan p;
+    KVHP_REQUIRE(cached_plan(rows, first, hq, hkv, d, p), KVHP_ERR_UNSUPPORTED,
+                 "prefill_cached: %d rows behind %d keys, heads %d/%d of %d", rows, first, hq, hkv, d);
+    KVHP_REQUIRE(ws_bytes >= prefill_cached_workspace(rows, first, hq, hkv, d), KVHP_ERR_WORKSPACE,
+                 "prefill_cached: workspace too small");
+    PrefillArgs a{};
+    a.q = static_cast<const f16*>(q);
+    a.k = static_cast<const f16*>(pool_k);
+    a.v = static_cast<const f16*>(pool_v);
+    a.out = static_cast<f16*>(out);
+    a.bt = bt;
+    a.max_pages = max_pages;
+    a.num_pages = num_pages;
+    a.S = rows;
+    a.Hq = hq;
+    a.Hkv = hkv;
+    a.G = hq / hkv;
+    a.RB = p.RB;
+    a.n_qblk = p.n_qblk;
+    a.scale_log2 = 1.4426950408889634f / std::sqrt(static_cast<float>(d));
+    a.HG = p.HG;
+    a.nsub = p.nsub;
+    a.first = first;
+    a.tiles_per_split = p.tiles;
+    a.nsplit = p.nsplit;
+    a.ws_o = static_cast<float*>(ws);
+    a.ws_ml = a.ws_o + (size_t)rows * hq * p.nsplit * d;
+    const dim3 grid(hkv * p.nsub * p.n_qblk, 1, p.nsplit);
+    if (d == 64)
+        hipLaunchKernelGGL((prefill_mfma_kernel<64, 2, true, true>), grid, dim3(8 * kWave), 0, s, a);
+    else
+        hipLaunchKernelGGL((prefill_mfma_kernel<128, 2, true, true>), grid, dim3(8 * kWave), 0, s, a);
+    const int rc = check_launch("prefill_cached");
+    if (rc || p.nsplit == 1) return rc;
+    const int64_t threads = (int64_t)rows * hq * (d / 8);
+    hipLaunchKernelGGL(prefill_merge_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)),
+                       dim3(256), 0, s, a.ws_o, a.ws_ml, a.out, threads, hq, d, first,
+                       p.tiles * kBN, p.nsplit);
+    return check_launch("prefill_cached (merge)");
 }
 
 }  // namespace kvhp
