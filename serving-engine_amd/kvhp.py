@@ -224,10 +224,25 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
-def _stream(stream) -> Optional[int]:
+def _current_stream() -> int:
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    return torch.cuda.current_stream().cuda_stream
+
+
+# The current stream's handle without building a torch.cuda.Stream object
+# around it (0.3 against 2.6 us, a third of a small call's host time).
+try:
+    from torch._C import _cuda_getCurrentRawStream, _cuda_getDevice
+except ImportError:
+    _cuda_getCurrentRawStream = None
+
+
+def _stream(stream) -> Optional[int]:
+    if stream is not None:
+        return stream.cuda_stream
+    if _cuda_getCurrentRawStream is None:
+        return _current_stream()
+    return _cuda_getCurrentRawStream(_cuda_getDevice())
 
 
 # ----------------------------------------------------------------- views --
