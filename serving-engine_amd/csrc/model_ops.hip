@@ -612,6 +612,22 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
         return a.y_tiles ? act_tiled_index(b, n, a.y_tiles) : (int64_t)b * a.ldy + n;
     };
 
+    // This thread's first output of a tile: batch row b0 (the same for every
+    // tile); for the QKV epilogue its write position, loaded ahead of
+    // everything else.
+    const int o0 = static_cast<int>(threadIdx.x);
+    const int b0 = 16 * (o0 / kOut) + (o0 & 15);
+    int pos0 = -1;
+    float rc = 1.f, rsn = 0.f;   // and its rotation
+    if constexpr (EPI == kEpiQKV) {
+        if (o0 < NBT * kOut && b0 < a.B) pos0 = a.positions[b0];
+    }
+    // RoPE rotation of output o of tile tl (QKV epilogue), at position pos.
+    auto rotation = [&](int tl, int o, int pos, float& c, float& sn) {
+        const int tph = a.D / L, hh = tl / tph, m = (o % kOut) >> 4;
+        if (hh < a.Hq + a.Hkv && m < P) rope_cs(pos < 0 ? 0 : pos, P * (tl % tph) + m, a.D, a.theta, c, sn);
+    };
+
     half8 wa[C], wb[C];
     int tile = static_cast<int>(blockIdx.x);
     if constexpr (kSeq) {
@@ -648,6 +664,14 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
         // every load above in flight before the first use (one round trip;
         // the scheduler would otherwise pair loads with their uses)
         __builtin_amdgcn_sched_barrier(0);
+        // The first tile's rotation while x and the weights land: behind the
+        // products powf, cosf and sinf added their latency to the launch (the
+        // 22-layer batched step 949 -> 930 us at B = 8, 1238 -> 1221 at 32).
+        if constexpr (EPI == kEpiQKV) {
+            if (o0 < NBT * kOut && b0 < a.B) rotation(tile, o0, pos0, rc, rsn);
+            asm volatile("" ::"v"(rc), "v"(rsn));
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (kStage && a.x_tiles == 0) {
             // into this wave's region (chunk c of row r at c ^ (r & 7): the
             // 8-lane phases of both the writes and the operand reads hit
@@ -707,22 +731,16 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
         }
     }
 
-    // This thread's first output of a tile: batch row b0 (the same for every
-    // tile); for the QKV epilogue its write position and page, loaded once.
-    const int o0 = static_cast<int>(threadIdx.x);
-    const int b0 = 16 * (o0 / kOut) + (o0 & 15);
-    int pos0 = -1, pid0 = -1;
+    // The page of this thread's first output's position (QKV epilogue).
+    int pid0 = -1;
     if constexpr (EPI == kEpiQKV) {
-        if (o0 < NBT * kOut && b0 < a.B) {
-            pos0 = a.positions[b0];
-            if (pos0 >= 0 && (pos0 >> 4) < a.max_pages)
-                pid0 = a.bt[(int64_t)b0 * a.max_pages + (pos0 >> 4)];
-        }
+        if (o0 < NBT * kOut && b0 < a.B && pos0 >= 0 && (pos0 >> 4) < a.max_pages)
+            pid0 = a.bt[(int64_t)b0 * a.max_pages + (pos0 >> 4)];
     }
 
     // Output o of a tile from its reduced sums; rv: the residual of that
-    // output (Residual epilogue).
-    auto epilogue = [&](int tl, int o, int rb, float rv, int pos, int pid) {
+    // output (Residual epilogue); (c, sn) its rotation (QKV).
+    auto epilogue = [&](int tl, int o, int rb, float rv, int pos, int pid, float c, float sn) {
         const int bt = o / kOut, rem = o % kOut, m = rem >> 4, n = rem & 15;
         const int b = 16 * bt + n;
         if (b >= a.B || m >= (kPair ? P : L)) return;
@@ -739,8 +757,6 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
             const float x1 = round16(v0), x2 = round16(v1);
             float o1 = x1, o2 = x2;
             if (hh < a.Hq + a.Hkv) {
-                float c, sn;
-                rope_cs(pos < 0 ? 0 : pos, d, a.D, a.theta, c, sn);
                 o1 = x1 * c - x2 * sn;
                 o2 = x2 * c + x1 * sn;
             }
@@ -783,6 +799,10 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
         if (pf && kDB) load_w(tl + G, nxt);
         if constexpr (!kDB) load_w(tl, cur);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (EPI == kEpiQKV) {   // the first tile's is there already
+            if (tl != static_cast<int>(blockIdx.x) && o0 < NBT * kOut && b0 < a.B)
+                rotation(tl, o0, pos0, rc, rsn);
+        }
         floatx4 acc[NBT];
         if constexpr (kSeq) {
 #pragma unroll
@@ -819,10 +839,10 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
         lds_barrier();
         for (int o = o0; o < NBT * kOut; o += static_cast<int>(blockDim.x)) {
             if (o == o0) {
-                epilogue(tl, o, rb, static_cast<float>(r0), pos0, pid0);
+                epilogue(tl, o, rb, static_cast<float>(r0), pos0, pid0, rc, rsn);
             } else {
                 const int b = 16 * (o / kOut) + (o & 15);
-                float rv = 0.f;
+                float rv = 0.f, c = 1.f, sn = 0.f;
                 int pos = -1, pid = -1;
                 if (b < a.B) {
                     if constexpr (EPI == kEpiResidual)
@@ -832,9 +852,10 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
                         pos = a.positions[b];
                         if (pos >= 0 && (pos >> 4) < a.max_pages)
                             pid = a.bt[(int64_t)b * a.max_pages + (pos >> 4)];
+                        rotation(tl, o, pos, c, sn);
                     }
                 }
-                epilogue(tl, o, rb, rv, pos, pid);
+                epilogue(tl, o, rb, rv, pos, pid, c, sn);
             }
         }
     };
