@@ -146,16 +146,9 @@ gemm_kernel(const GemmArgs a) {
         const int row = r < BN ? wrow(r) : min(m0 + r - BN, a.M - 1);
         voff[p] = static_cast<uint32_t>(row) * static_cast<uint32_t>(2 * a.K) + 16 * c;
     }
-    // Each XCD starts its walk over K at another step: in step, all of them
-    // would read the same columns of every row at once (the 22-layer decoder's
-    // prompts of 700 / 1024 / 2048 tokens 3405 / 3780 / 5618 us in step, 3308 /
-    // 3650 / 5575 so; the sums' order is fixed by the shape).
-    const int rot = static_cast<int>(blockIdx.x & 7) * KT / 8;
     auto issue = [&](int slot, int t, int p) {   // load p of step t
         const int inst = wave * LPT + p;         // uniform
-        int kt = t + rot;
-        if (kt >= KT) kt -= KT;
-        const f16* base = (inst * RPI < BN ? a.W : a.A) + (k0 + kt) * BK;
+        const f16* base = (inst * RPI < BN ? a.W : a.A) + (k0 + t) * BK;
         dma16s(base, voff[p], ring0 + (slot * STG + inst * RPI * BK) * 2);
     };
     // operand reads: rows of this wave's tiles at chunk 2q + h of piece q
