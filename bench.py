@@ -901,7 +901,7 @@ def run_config5(torch, kvhp, steps=128, prompt_len=2048):
     cfg = kvhp.llama_1b_config()
     model = kvhp.LlamaModel(cfg, seed=5, max_ctx=prompt_len + steps + 1)
     prompt = np.random.default_rng(5).integers(0, cfg.vocab_size, prompt_len).astype(np.int32)
-    model.prefill(prompt[:16])                     # warm the library paths (rocBLAS, kernels)
+    model.prefill(prompt[:16])                     # warm the library paths (kernels)
     model.close()
     model = kvhp.LlamaModel(cfg, seed=5, max_ctx=prompt_len + steps + 1)
     t0 = time.perf_counter()

@@ -496,7 +496,8 @@ int kvhp_llama_prefill_cached(void* model, const int32_t* tokens, int n, int num
  * step, from the model's tiled copy of it, which the first such step builds
  * on `stream` -- as large as the four projections and the LM head; weights
  * written through kvhp_llama_tensor after that are seen by batched steps once
- * kvhp_llama_reserve rebuilds the copies); larger batches on library GEMMs.
+ * kvhp_llama_reserve rebuilds the copies); larger batches on the
+ * prompt's MFMA projections.
  * Asynchronous on `stream`. */
 int kvhp_llama_decode_paged(void* model, const int32_t* tokens, int batch, void* pool,
                             int num_pages, const int32_t* block_tables, int max_pages,
@@ -513,7 +514,8 @@ int kvhp_llama_decode_paged(void* model, const int32_t* tokens, int batch, void*
  * so graphs captured earlier keep valid addresses); under HIP graph capture it
  * cannot, and returns KVHP_ERR_WORKSPACE having enqueued at most the step's
  * embedding lookup.  So: reserve before capturing decode_paged (batches up to
- * 32; larger batches run library GEMMs, which are not meant for capture).
+ * 32; larger batches run the prompt's projections, some sizes of which are
+ * library GEMMs: not meant for capture).
  * kvhp_llama_prefill_paged / _cached synchronise and are never captured. */
 int kvhp_llama_reserve(void* model, int max_batch, int max_seq_len);
 

@@ -20,10 +20,11 @@
 // up rows, RoPE dims d / d + D/2), so both members of a pair meet in one lane.
 //
 // A step is four quarters of 16 of K; a wave reads the next quarter's operands
-// while the MFMAs of this one run.  Before the last quarter's MFMAs it waits for
-// its own loads of step t+1, meets the workgroup (every wave is done reading
-// step t, and step t+1 has landed), loads step t+NS over step t and reads the
-// first quarter of step t+1.
+// while the MFMAs of this one run, and over the first three quarters loads step
+// t+NS-1 into the slot of step t-1.  Before the last quarter's MFMAs it waits
+// for its own loads of step t+1 and meets the workgroup (every wave is done
+// reading step t, and step t+1 has landed), then reads the first quarter of
+// step t+1.
 #include "kvhp_internal.h"
 
 #include <algorithm>

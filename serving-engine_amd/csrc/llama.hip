@@ -438,8 +438,8 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
 // positions[b] (its K/V appended there through row b of pg.bt) and attends
 // over seq_lens[b] keys; fp32 logits [B][V], greedy tokens next[b].  One row
 // runs on the batch-1 step's GEMV kernels, up to 32 on the fused skinny-GEMM
-// kernels, larger batches on library GEMMs with separate RMSNorm / RoPE /
-// SwiGLU launches.
+// kernels, larger batches on the prompt's projections (gemm.hip), RMSNorm a
+// launch of its own.
 // Tiled copies of the projection weights for the batched kernels (each weight
 // load 1 KB contiguous; bit-identical outputs): allocated once, (re)written
 // from the row-major weights on stream s.  Not under graph capture (an

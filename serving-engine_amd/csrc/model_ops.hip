@@ -22,9 +22,9 @@
 // past K or by slabs; a generic one-wave-per-row kernel covers other K and
 // unaligned operands.
 //
-// Prefill uses library GEMMs (rocBLAS) for the projections; the row-wise
-// RMSNorm, the RoPE that also splits the fused QKV output, and SwiGLU over
-// the fused gate|up output are here.  Greedy sampling is an on-device argmax
+// Prompt projections are gemm.hip's; the row-wise RMSNorm, and the RoPE that
+// also splits the fused QKV output and SwiGLU over the fused gate|up output
+// for projections that run without them in the epilogue, are here.  Greedy sampling is an on-device argmax
 // with the lowest index winning ties (the reference's host loop,
 // generate.cpp:714-721), which also advances the device-side sequence length
 // so that a captured decode step needs no host round trip.
@@ -884,7 +884,7 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
 
 // Slice shape for K: C = 8 (8 x 16 bytes per lane and row) with K/256 <= 8
 // waves, or C = 11 with K/352 <= 16 waves (K = 5632: 16 waves).  Other K, or
-// B > 32: unsupported (the caller keeps the library GEMM).
+// B > 32: unsupported (the caller takes the prompt's projections).
 bool rows_shape(int K, int& C, int& NW) {
     if (K % 256 == 0 && K / 256 >= 1 && K / 256 <= 8) {
         C = 8;

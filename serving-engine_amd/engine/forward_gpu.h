@@ -14,7 +14,7 @@
 // [L][2][Hkv][max_seq][D] block is read as a page pool [L][2][Hkv][P][16][D]
 // through an identity block table (byte-identical for max_seq = 16 P, so
 // max_seq must be a multiple of 16), prefill runs kvhp_llama_prefill_paged
-// (library GEMMs + the flash prefill kernel writing the pages) and a decode
+// (MFMA projections + the flash prefill kernel writing the pages) and a decode
 // step kvhp_llama_decode_paged (fused GEMVs, split-K decode attention).
 //
 // Differences by design:
@@ -24,8 +24,8 @@
 //     reference's loader, outside the KV-cache path; tie_word_embeddings
 //     copies the embedding into the LM head.  It also owns the model's
 //     activation rows (max_rows, the longest prompt one prefill takes).
-//   * The BLAS handle is opaque and unused (the model owns its rocBLAS
-//     handle); any pointer, or nullptr, may be passed where the reference
+//   * The BLAS handle is opaque and unused (the model owns one
+//     where it needs it); any pointer, or nullptr, may be passed where the reference
 //     passes its cublasHandle_t.
 //   * profile_records, when given, receives one record per call (the
 //     call's device time), not one per kernel.
