@@ -755,15 +755,17 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
             const int tph = a.D / L;
             const int hh = tl / tph, d = P * (tl % tph) + m, half = a.D / 2;
             const float x1 = round16(v0), x2 = round16(v1);
-            float o1 = x1, o2 = x2;
+            // rounded where they are computed, so that the fused multiply-add
+            // rounds to fp16 once, as in the batch-1 kernel
+            f16 o1 = static_cast<f16>(x1), o2 = static_cast<f16>(x2);
             if (hh < a.Hq + a.Hkv) {
-                o1 = x1 * c - x2 * sn;
-                o2 = x2 * c + x1 * sn;
+                o1 = static_cast<f16>(x1 * c - x2 * sn);
+                o2 = static_cast<f16>(x2 * c + x1 * sn);
             }
             if (hh < a.Hq) {
                 f16* q = a.y16 + (int64_t)b * a.ldy + hh * a.D;
-                q[d] = static_cast<f16>(o1);
-                q[d + half] = static_cast<f16>(o2);
+                q[d] = o1;
+                q[d + half] = o2;
                 return;
             }
             if (pid < 0 || pid >= a.num_pages) return;
@@ -771,8 +773,8 @@ __global__ void __launch_bounds__(kWave * NWMAX) gemm_rows_kernel(const RowsArgs
             const int kvh = isk ? hh - a.Hq : hh - a.Hq - a.Hkv;
             f16* dst = (isk ? a.pool_k : a.pool_v) +
                        (((int64_t)kvh * a.num_pages + pid) * kPage + (pos & 15)) * a.D;
-            dst[d] = static_cast<f16>(o1);
-            dst[d + half] = static_cast<f16>(o2);
+            dst[d] = o1;
+            dst[d + half] = o2;
         } else if constexpr (EPI == kEpiSwiglu) {
             const int nn = P * tl + m;
             if (nn < a.N) a.y16[yat(b, nn)] = static_cast<f16>(silu_mul(round16(v0), round16(v1)));
