@@ -76,11 +76,23 @@ __device__ __forceinline__ void stage_barrier() {
 
 __device__ __forceinline__ float r16(float v) { return static_cast<float>(static_cast<f16>(v)); }
 
-// silu(g) u on the hardware's exponential and reciprocal (1 ulp each; the
-// product is rounded to fp16 next).  expf and the IEEE division took 4 us of a
-// 256 x 128 tile's time.
+// silu(g) u for a gate rounded to fp16: the bits of g / (1 + expf(-g)) u at all
+// 65536 gates, on half the instructions.  The exponent -g log2(e) is an exact
+// product (g has 11 bits, the constant's head 13) plus the rest of the constant;
+// the quotient is a reciprocal's product and one residual step, in sixteenths so
+// that no reciprocal is subnormal.  Where the residual is zero, or NaN (infinite
+// gates and exponentials), the product stands.  A 2048-id prompt of the 22-layer
+// 2048 / 5632 model takes 5508 us, and 2.7 % (against 1.4 %) over that of
+// v_exp_f32 of the rounded product and v_rcp_f32 with expf and the IEEE division;
+// those two alone are up to 61 units of 2^-24 off, expf and this 2.4.
 __device__ __forceinline__ float silu_mul(float g, float u) {
-    return g * __builtin_amdgcn_rcpf(1.f + fast_exp2(-1.4426950408889634f * g)) * u;
+    constexpr float hi = -1.442626953125f, lo = static_cast<float>(-1.4426950408889634 - hi);
+    const float gc = __builtin_amdgcn_fmed3f(g, -200.f, 200.f);   // exp(-g) infinite or 0 beyond
+    const float t = gc * hi, n = rintf(t);
+    const float e = ldexpf(fast_exp2(fmaf(gc, lo, t - n)), static_cast<int>(n));
+    const float d = fmaf(e, 0.0625f, 0.0625f), g16 = g * 0.0625f;
+    const float r = __builtin_amdgcn_rcpf(d), q = g16 * r, res = fmaf(-d, q, g16);
+    return (__builtin_islessgreater(res, 0.f) ? fmaf(res, r, q) : q) * u;
 }
 
 template <int BN, int BM, int BK, int WN, int WM, int NS, int EPI>
