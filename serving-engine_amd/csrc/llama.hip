@@ -166,24 +166,26 @@ int regrow(Model& m, T** p, size_t* cap, size_t n, hipStream_t s, const char* wh
     return KVHP_OK;
 }
 
-// Decode-attention workspace for B sequences of up to max_seq_len keys,
-// owned by the model (not the library's per-device buffer), so that models
-// on different streams never share split partials.
-// With `bytes_needed` that size instead (the cached-prefix attention's partials).
-int rows_workspace(Model& m, int B, int max_seq_len, hipStream_t s, void** ws, size_t* bytes,
-                   size_t bytes_needed = 0) {
-    const kvhp_llama_config& c = m.c;
-    const size_t need = bytes_needed ? bytes_needed
-                                     : kvhp_decode_workspace_bytes(B, c.num_q_heads, c.num_kv_heads,
-                                                                   c.head_dim, max_seq_len, 0);
+// `need` bytes of attention workspace, owned by the model (not the library's
+// per-device buffer), so that models on different streams never share split
+// partials.  0 bytes grow nothing.
+int attn_workspace(Model& m, size_t need, hipStream_t s, void** ws, size_t* bytes) {
     if (need > m.ws_rows_bytes) {
         char* p = static_cast<char*>(m.ws_rows);
-        KVHP_TRY(regrow(m, &p, &m.ws_rows_bytes, need, s, "decode-attention workspace"));
+        KVHP_TRY(regrow(m, &p, &m.ws_rows_bytes, need, s, "attention workspace"));
         m.ws_rows = p;
     }
     *ws = m.ws_rows;
     *bytes = m.ws_rows_bytes;
     return KVHP_OK;
+}
+
+// That of a decode step over B sequences of up to max_seq_len keys.
+int rows_workspace(Model& m, int B, int max_seq_len, hipStream_t s, void** ws, size_t* bytes) {
+    const kvhp_llama_config& c = m.c;
+    return attn_workspace(m, kvhp_decode_workspace_bytes(B, c.num_q_heads, c.num_kv_heads,
+                                                         c.head_dim, max_seq_len, 0),
+                          s, ws, bytes);
 }
 
 int blas_check(rocblas_status st, const char* what) {
@@ -405,8 +407,11 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
     void* ws = nullptr;
     size_t ws_bytes = 0;
     const bool flash = prefill_cached_fits(S, first, Hq, Hkv, D) && aligned16(pg.base);
-    KVHP_TRY(rows_workspace(m, S, n, s, &ws, &ws_bytes,
-                            flash ? prefill_cached_workspace(S, first, Hq, Hkv, D) : 0));
+    if (flash)   // 0 when a block's keys are one split
+        KVHP_TRY(attn_workspace(m, prefill_cached_workspace(S, first, Hq, Hkv, D), s, &ws,
+                                &ws_bytes));
+    else
+        KVHP_TRY(rows_workspace(m, S, n, s, &ws, &ws_bytes));
     const Pages rows_pg{pg.base, pg.num_pages, sr.tables, pg.max_pages};
     KVHP_TRY(forward_rope(m, S, first, nullptr, s));
     KVHP_TRY(kvhp_embedding(m.tokens + first, m.embed, m.hidden, S, H, c.vocab_size, s));
