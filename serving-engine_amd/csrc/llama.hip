@@ -344,17 +344,18 @@ int prefill_layers(Model& m, int n, const Pages& pg, void* s) {
     return KVHP_OK;
 }
 
-// Inputs of a cached-prefix prefill's attention, on the device: row r of
-// tables [rows][width] is the sequence's block-table row, lens[r] =
-// first + r + 1 (query row r sits at position first + r), start[0] = first.
+// Inputs of a cached-prefix prefill, on the device: start[0] = first, and for
+// suffix rows taken as rows of a decode step (rows > 0) lens[r] = first + r + 1,
+// pos[r] = first + r and row r of tables (and wtables) [rows][width] the
+// sequence's read (write) block-table row.  Null tables are not written.
 __global__ void suffix_rows_kernel(int32_t* tables, int32_t* wtables, int32_t* lens,
                                    int32_t* pos, int32_t* start, const int32_t* row,
                                    const int32_t* wrow, int rows, int width, int first) {
     const int64_t total = (int64_t)rows * width;
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * blockDim.x) {
-        tables[i] = row[i % width];
-        wtables[i] = wrow[i % width];
+        if (tables) tables[i] = row[i % width];
+        if (wtables) wtables[i] = wrow[i % width];
     }
     for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < rows;
          r += (int64_t)gridDim.x * blockDim.x) {
@@ -364,23 +365,29 @@ __global__ void suffix_rows_kernel(int32_t* tables, int32_t* wtables, int32_t* l
     if (blockIdx.x == 0 && threadIdx.x == 0) start[0] = first;
 }
 
-// Device inputs of a cached-prefix prefill of `rows` suffix rows (in m.aux):
-// replicated read and write block-table rows, lengths, positions, start.
+// Those inputs (in m.aux) for a suffix of `rows` rows: what its route reads.
 struct SuffixRows {
     int32_t *tables, *wtables, *lens, *pos, *start;
 };
+enum SuffixRoute {
+    kSuffixFlash,    // attention on the sequence's own block-table row: start only
+    kSuffixAttend,   // attention as rows of a decode call: lengths and read tables too
+    kSuffixStep,     // a batched decode step: write tables as well
+};
 
 int suffix_rows(Model& m, const Pages& pg, const int32_t* write_bt, int first, int rows,
-                hipStream_t s, SuffixRows& out) {
-    const size_t words = 2 * (size_t)rows * pg.max_pages + 2 * (size_t)rows + 1;
+                SuffixRoute route, hipStream_t s, SuffixRows& out) {
+    if (route == kSuffixFlash) rows = 0;
+    const size_t table = (size_t)rows * pg.max_pages;
+    const size_t words = table * (route == kSuffixStep ? 2 : 1) + 2 * (size_t)rows + 1;
     if (m.aux_words < words)
         KVHP_TRY(regrow(m, &m.aux, &m.aux_words, words, s, "suffix block tables"));
-    out.tables = m.aux;
-    out.wtables = out.tables + (size_t)rows * pg.max_pages;
-    out.lens = out.wtables + (size_t)rows * pg.max_pages;
+    out.tables = route == kSuffixFlash ? nullptr : m.aux;
+    out.wtables = route == kSuffixStep ? m.aux + table : nullptr;
+    out.lens = m.aux + table * (route == kSuffixStep ? 2 : 1);
     out.pos = out.lens + rows;
     out.start = out.pos + rows;
-    const int64_t blocks = std::min<int64_t>(((int64_t)rows * pg.max_pages + 255) / 256, 1024);
+    const int64_t blocks = std::min<int64_t>(((int64_t)table + 255) / 256 + 1, 1024);
     hipLaunchKernelGGL(suffix_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s,
                        out.tables, out.wtables, out.lens, out.pos, out.start, pg.bt, write_bt,
                        rows, pg.max_pages, first);
@@ -400,13 +407,11 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
     const int H = c.hidden_size, D = c.head_dim, Hq = c.num_q_heads, Hkv = c.num_kv_heads;
     const int F = c.ffn_size;
     const int S = n - first;
+    const bool flash = prefill_cached_fits(S, first, Hq, Hkv, D) && aligned16(pg.base);
     SuffixRows sr{};
-    KVHP_TRY(suffix_rows(m, pg, write_bt, first, S, s, sr));
-    int32_t* lens = sr.lens;
-    int32_t* start = sr.start;
+    KVHP_TRY(suffix_rows(m, pg, write_bt, first, S, flash ? kSuffixFlash : kSuffixAttend, s, sr));
     void* ws = nullptr;
     size_t ws_bytes = 0;
-    const bool flash = prefill_cached_fits(S, first, Hq, Hkv, D) && aligned16(pg.base);
     if (flash)   // 0 when a block's keys are one split
         KVHP_TRY(attn_workspace(m, prefill_cached_workspace(S, first, Hq, Hkv, D), s, &ws,
                                 &ws_bytes));
@@ -420,7 +425,7 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
         KVHP_TRY(kvhp_rmsnorm(m.hidden, L.attn_norm, m.norm, S, H, c.rms_eps, s));
         KVHP_TRY(project_qkv(m, L, S, first, nullptr, s));
         KVHP_TRY(kvhp_paged_append_kv(m.k, m.v, layer_pool(m, pg, l, 0), layer_pool(m, pg, l, 1),
-                                      write_bt, pg.max_pages, start, 1, S, Hkv, D, pg.num_pages,
+                                      write_bt, pg.max_pages, sr.start, 1, S, Hkv, D, pg.num_pages,
                                       s));
         if (flash) {
             KVHP_TRY(prefill_cached(m.q, layer_pool(m, pg, l, 0), layer_pool(m, pg, l, 1), pg.bt,
@@ -428,7 +433,7 @@ int prefill_suffix_layers(Model& m, int first, int n, const Pages& pg, const int
                                     ws_bytes, s));
         } else {
             const kvhp_kv_view kv = pages_view(m, rows_pg, l, 0), vv = pages_view(m, rows_pg, l, 1);
-            KVHP_TRY(kvhp_decode_attention(m.q, &kv, &vv, lens, m.attn, S, Hq, Hkv, D, n, 0, ws,
+            KVHP_TRY(kvhp_decode_attention(m.q, &kv, &vv, sr.lens, m.attn, S, Hq, Hkv, D, n, 0, ws,
                                            ws_bytes, s));
         }
         KVHP_TRY(project_residual(m, m.attn, L.w_o, S, Hq * D, s));
@@ -884,7 +889,8 @@ int prefill_pages(void* model, const int32_t* tokens, int n, int first, void* po
         // a short suffix is one batched decode step: row r at position
         // first + r appends its K/V, then attends over first + r + 1 keys
         SuffixRows sr{};
-        KVHP_TRY(suffix_rows(m, pg, write_table ? write_table : block_table, first, S, s, sr));
+        KVHP_TRY(suffix_rows(m, pg, write_table ? write_table : block_table, first, S,
+                             kSuffixStep, s, sr));
         const Pages rows_pg{pg.base, pg.num_pages, sr.tables, pg.max_pages};
         KVHP_TRY(decode_rows(m, m.tokens + first, S, rows_pg, sr.pos, sr.lens, n,
                              m.suffix_logits, m.suffix_next, s, sr.wtables));

@@ -1,5 +1,6 @@
 """Device memory that a prompt behind a cached prefix takes beyond its model's: the
-flash route with one split of the keys needs no attention partials.
+flash route with one split of the keys needs no attention partials, and no copy of
+the block tables for each row.
 """
 import numpy as np
 import pytest
@@ -38,3 +39,10 @@ def test_one_split_takes_no_partials():
     4 x 2048 x 32 x 66 floats, 69 MB."""
     note("cached prompt: 2048 rows behind 2048 keys, memory")
     assert _grown(4096, 2048, 256) < 24 << 20
+
+
+def test_no_tables_per_row():
+    """2048 rows with tables of 4096 pages: a read and a write table a row are
+    2 x 2048 x 4096 words, 67 MB."""
+    note("cached prompt: 2048 rows with tables of 4096 pages, memory")
+    assert _grown(4096, 2048, 4096) < 24 << 20
