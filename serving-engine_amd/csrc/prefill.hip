@@ -184,7 +184,14 @@ __device__ __forceinline__ float halves_sum(float x) {
 // would wait for every DMA in flight).  Few query rows leave CUs idle, so the
 // keys may be cut into nsplit ranges; a row whose keys reach past the first
 // stores its partial (m, l, O) for prefill_merge_kernel.
-constexpr int kMaxTablePages = 4096;   // page ids of a split in LDS (65536 keys)
+// P is 0 at the keys past a row, but 0 times an infinite or NaN V is NaN, and a
+// later position's V must not reach an earlier row (whose K/V stay in pages that
+// other prompts share).  In the tiles that the causal mask can cut, such elements
+// are set to 0 in LDS, by the wave that loaded them, and added as they are at the
+// end to the rows at or past their key.  (The whole-prompt kernel does not: there
+// a non-finite V also reaches the earlier rows of its block.)
+constexpr int kMaxTablePages = 4088;   // page ids of a split in LDS (65408 keys) ...
+constexpr int kBadWords = 8;           // ... and the keys of 4 tiles with such a V
 
 template <int D, int KG, bool SUB, bool CACHED>
 __global__ void __launch_bounds__(8 * kWave)
@@ -210,7 +217,8 @@ prefill_mfma_kernel(const PrefillArgs a) {
 
     constexpr int NSTAGE = 4;
     __shared__ __attribute__((aligned(16))) f16 ring[NSTAGE * 2 * TB];
-    __shared__ int32_t ptab[CACHED ? kMaxTablePages : 1];
+    __shared__ int32_t ptab[CACHED ? kMaxTablePages + kBadWords : 1];
+    uint32_t* bad_keys = reinterpret_cast<uint32_t*>(ptab + kMaxTablePages);   // CACHED
 
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS bases in SGPRs
@@ -374,6 +382,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
                 const int pid = t_lo * 4 + i < a.max_pages ? a.bt[t_lo * 4 + i] : 0;
                 ptab[i] = min(max(pid, 0), a.num_pages - 1);
             }
+            if (tid < kBadWords) bad_keys[tid] = 0;
             __syncthreads();
             pid_next = ptab[page_of(0) - t_lo * 4];
         }
@@ -513,8 +522,35 @@ prefill_mfma_kernel(const PrefillArgs a) {
                     l_part = __builtin_amdgcn_fdot2(half2v{pop[t][e], pop[t][e + 1]}, ones, l_part,
                                                     false);
         };
+        // CACHED: from tile cut0 on the causal mask can cut a tile (at most 3 of
+        // the block's); this wave's rows of it, just landed, lose the elements of V
+        // that are not finite.
+        const int cut0 = (first + q0) / kBN - t_lo;
+        auto clean = [&](int j) {
+            f16* Vt = ring + (j % NSTAGE) * 2 * TB + TB + wave * IPW * RPI * D + 8 * lane;
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int p = 0; p < IPW; ++p) {
+                u32x4 x = *reinterpret_cast<const u32x4*>(Vt + p * RPI * D);
+                uint32_t m[4], any = 0;   // bits 15 / 31: an exponent of all ones
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    m[i] = ((x[i] & 0x7fff7fffu) + 0x04000400u) & 0x80008000u;
+                    any |= m[i];
+                }
+                if (any == 0) continue;
+                const int r = (wave * IPW + p) * RPI + lane / CPR;
+                atomicOr(&bad_keys[2 * (j - cut0) + (r >> 5)], 1u << (r & 31));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] &= ~(m[i] | (m[i] - (m[i] >> 15)));
+                *reinterpret_cast<u32x4*>(Vt + p * RPI * D) = x;
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): written before the barrier
+        };
         auto phase_start = [&](int j) {   // barrier into phase 2j, then tile j+2
             wait_vmcnt<LPT>();
+            if (CACHED && j >= cut0 && j < n_tiles) clean(j);
             ring_barrier();
             const int tt = j + 2;
             issue(ring + (tt % NSTAGE) * 2 * TB, tt);
@@ -618,6 +654,33 @@ prefill_mfma_kernel(const PrefillArgs a) {
                         for (int e = 0; e < 4; ++e)
                             o[db][4 * q4 + e] = o[db][4 * q4 + e] * a0 + v4[e] * a1;
                     }
+            }
+        }
+
+        if constexpr (CACHED) {
+            // ---- the V elements left out above, from the pages
+            uint32_t any = 0;
+#pragma unroll
+            for (int i = 0; i < kBadWords; ++i) any |= bad_keys[i];
+            if (__builtin_amdgcn_readfirstlane(any) && kgrp == 0) {
+#pragma unroll 1
+                for (int i = 0; i < 32 * kBadWords; ++i) {
+                    const int key = (t_lo + cut0) * kBN + i;
+                    if (!(bad_keys[i >> 5] >> (i & 31) & 1) || key >= n_keys) continue;
+                    const f16* src = vb + ((int64_t)ptab[(key >> 4) - t_lo * 4] * kPage + key % kPage) * D + 4 * h;
+#pragma unroll
+                    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                        for (int q4 = 0; q4 < 4; ++q4) {
+                            const half4 v = *reinterpret_cast<const half4*>(src + 32 * db + 8 * q4);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const float x = static_cast<float>(v[e]);
+                                if (key <= first + row && !(fabsf(x) < INFINITY))
+                                    o[db][4 * q4 + e] += x;
+                            }
+                        }
+                }
             }
         }
 
