@@ -224,25 +224,19 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
-def _current_stream() -> int:
-    import torch
-    return torch.cuda.current_stream().cuda_stream
-
-
-# The current stream's handle without building a torch.cuda.Stream object
-# around it (0.3 against 2.6 us, a third of a small call's host time).
-try:
-    from torch._C import _cuda_getCurrentRawStream, _cuda_getDevice
-except ImportError:
-    _cuda_getCurrentRawStream = None
-
-
 def _stream(stream) -> Optional[int]:
     if stream is not None:
         return stream.cuda_stream
-    if _cuda_getCurrentRawStream is None:
-        return _current_stream()
-    return _cuda_getCurrentRawStream(_cuda_getDevice())
+    import torch   # here, so that importing this module loads no torch
+    # The current stream's handle without building a torch.cuda.Stream object
+    # around it (0.4 against 2.8 us, a third of a small call's host time), once
+    # torch has initialised the device (never in a forked child, which it refuses).
+    if torch.cuda.is_initialized():
+        try:
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:   # not public names
+            pass
+    return torch.cuda.current_stream().cuda_stream
 
 
 # ----------------------------------------------------------------- views --
