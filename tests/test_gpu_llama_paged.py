@@ -169,8 +169,8 @@ def test_paged_runner_matches_batch1_runner_and_oracle():
 
 @pytest.mark.parametrize("ffn", [1024, 5632])
 def test_paged_runner_large_batch_path_matches_fused_path(ffn):
-    """Batches above 32 run on library GEMMs with separate norm / RoPE /
-    SwiGLU launches; up to 32 on the fused batched projections.  One step
+    """Batches above 32 run on the prompt's MFMA projections with a norm
+    launch of its own; up to 32 on the fused batched projections.  One step
     of 40 sequences on one copy of the pool against the same step as two
     calls of 20 on another copy: logits within 2% of the scale, tokens equal
     outside near-ties, and the appended K/V rows within fp16 rounding.  With
@@ -246,8 +246,8 @@ def test_paged_runner_single_sequence_step_is_the_batch1_step():
 def test_cached_prefix_prefill_matches_full_prefill(suffix):
     """kvhp_llama_prefill_cached over a prefix whose K/V another prefill
     wrote: up to 32 suffix rows run as one batched decode step (one row on
-    the batch-1 kernels), longer suffixes layer by layer with a batched
-    decode-attention call; either way the last position's logits match the
+    the batch-1 kernels), longer suffixes layer by layer with the flash
+    kernel over the pages; either way the last position's logits match the
     whole-prompt prefill within 2 % of the scale (near-tie rule for the
     token), the prefix pages keep their bytes and the suffix K/V land in the
     following pages."""
@@ -285,8 +285,9 @@ def test_paged_runner_qwen_shapes_use_the_fallback_projections():
     """The reference runner's own model shapes (docs/runner_interface.md:
     hidden 896, 14 query / 2 KV heads -- G = 7 --, head_dim 64; here 2
     layers, FFN 4864, vocab 3000): hidden 896 is not a multiple of 256, so
-    batches of 2..32 take the library-GEMM path and a batch of one the
-    generic batch-1 GEMVs.  Three sequences, prefill and four decode steps,
+    batches of 2..32 take the prompt's MFMA projections and a batch of one the
+    batch-1 GEMVs with masked chunks (K = 896) and slabs (K = 4864); the head
+    of 3000 columns is the library's product.  Three sequences, prefill and four decode steps,
     against batch-1 models of the same weights (2 % of the logit scale,
     near-tie rule)."""
     cfg = kvhp.LlamaConfig(3000, 896, 2, 14, 2, 64, 4864, 1e-6, 1000000.0, 0)
@@ -305,7 +306,7 @@ def test_paged_runner_qwen_shapes_use_the_fallback_projections():
         assert tok == rtok and np.array_equal(lg, rlg), f"prefill {i}"
         toks.append(tok)
     seq = [len(p) for p in prompts]
-    for B in (3, 1):                      # library GEMMs, then the batch-1 kernels
+    for B in (3, 1):                      # the prompt's projections, then the batch-1 kernels
         for step in range(2):
             logits = torch.empty(B, V, dtype=torch.float32, device="cuda")
             nxt = torch.empty(B, dtype=torch.int32, device="cuda")

@@ -4,7 +4,9 @@ over K: logits and the K/V pages of every layer against the same forward in 64
 bits on the GPU (plain torch).  The forward rounds activations to fp16 after every
 operator (2^-11 relative each, independent): through two layers the relative
 2-norm error stays below 2e-3, and the batched step's too; 4e-3 is asserted.  A
-tile read or written in the wrong place is an error of order 1.
+tile read or written in the wrong place is an error of order 1.  Dimensions that
+those kernels do not take run on the library's products with the row-wise operators
+between them, and are held to the same.
 """
 import math
 
@@ -18,15 +20,24 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-# hidden 576 = 9 heads of 64 (tile tails in N), ffn 1472 = 23 steps of 64; heads of 128
+# hidden 576 = 9 heads of 64 (tile tails in N), ffn 1472 = 23 steps of 64; heads of 128;
+# ffn 4864 = 76 steps: 8 ranges of K, the last one shorter
 CONFIGS = {
     "d64": (544, 576, 2, 9, 3, 64, 1472),
     "d128": (512, 1024, 2, 8, 2, 128, 2816),
+    "ffn4864": (544, 576, 2, 9, 3, 64, 4864),
+}
+# on the library's products: heads of 32; ffn not a multiple of 64 (attention behind a
+# cached prefix on the flash route); a vocabulary not a multiple of 32 (the head alone)
+LIBRARY = {
+    "d32": (544, 512, 2, 16, 4, 32, 1408),
+    "ffn1440": (544, 512, 2, 8, 2, 64, 1440),
+    "vocab550": (550, 576, 2, 9, 3, 64, 1472),
 }
 
 
 def _model(name, max_ctx):
-    v, h, layers, hq, hkv, d, f = CONFIGS[name]
+    v, h, layers, hq, hkv, d, f = {**CONFIGS, **LIBRARY}[name]
     return kvhp.LlamaModel(kvhp.LlamaConfig(v, h, layers, hq, hkv, d, f, 1e-5, 10000.0, 0), 3,
                            max_ctx)
 
@@ -86,37 +97,60 @@ def _pages(m, n, extra=0):
     return pool, p
 
 
+def _check_prompt(m, ref, rng, name, n, first=0):
+    """A prompt of n ids, its positions below `first` cached by another call."""
+    note(f"prompt gemm {name} n={n} first={first}")
+    ids = rng.integers(0, m.config.vocab_size, n).astype(np.int32)
+    want, cache = ref.prompt(ids)
+    pool, p = _pages(m, n, extra=1)
+    perm = rng.permutation(p - 1).astype(np.int32)
+    bt = torch.from_numpy(perm).cuda()
+    if first:
+        m.prefill_paged(ids[:first], pool, p, bt, p - 1)
+        _, logits = m.prefill_cached(ids, first, pool, p, bt, p - 1)
+    else:
+        _, logits = m.prefill_paged(ids, pool, p, bt, p - 1)
+    assert _rel(torch.from_numpy(logits).cuda(), want) < 4e-3
+    rows = (bt.long()[:, None] * 16 + torch.arange(16, device="cuda")).reshape(-1)[:n]
+    for l in range(m.config.num_layers):
+        for kv in range(2):
+            got = pool[l, kv].reshape(m.config.num_kv_heads, -1, m.config.head_dim)[:, rows]
+            assert _rel(got, cache[l][kv]) < 4e-3, (n, l, kv)
+    assert not bool(pool[:, :, :, p - 1].any())        # the page outside the table
+
+
 @pytest.mark.parametrize("name", sorted(CONFIGS))
 def test_prompt_rows_at_tile_edges(name):
     m = _model(name, 1100)
     ref = _Ref(m)
     rng = np.random.default_rng(4)
     for n in (1, 2, 31, 33, 63, 64, 65, 127, 129, 192, 257, 500, 513, 1030):
-        note(f"prompt gemm {name} n={n}")
-        ids = rng.integers(0, m.config.vocab_size, n).astype(np.int32)
-        want, cache = ref.prompt(ids)
-        pool, p = _pages(m, n, extra=1)
-        perm = rng.permutation(p - 1).astype(np.int32)
-        bt = torch.from_numpy(perm).cuda()
-        _, logits = m.prefill_paged(ids, pool, p, bt, p - 1)
-        assert _rel(torch.from_numpy(logits).cuda(), want) < 4e-3
-        rows = (bt.long()[:, None] * 16 + torch.arange(16, device="cuda")).reshape(-1)[:n]
-        for l in range(m.config.num_layers):
-            for kv in range(2):
-                got = pool[l, kv].reshape(m.config.num_kv_heads, -1, m.config.head_dim)[:, rows]
-                assert _rel(got, cache[l][kv]) < 4e-3, (n, l, kv)
-        assert not bool(pool[:, :, :, p - 1].any())        # the page outside the table
+        _check_prompt(m, ref, rng, name, n)
     m.close()
 
 
-def test_large_batch_step():
+@pytest.mark.parametrize("name", sorted(LIBRARY))
+def test_prompt_on_library_products(name):
+    """Whole prompts and prompts behind a cached prefix."""
+    m = _model(name, 300)
+    ref = _Ref(m)
+    rng = np.random.default_rng(6)
+    for n, first in ((1, 0), (2, 0), (33, 0), (130, 0), (300, 0), (60, 20), (131, 16), (300, 200)):
+        _check_prompt(m, ref, rng, name, n, first)
+    m.close()
+
+
+@pytest.mark.parametrize("name,shift", [("d64", 0), ("d64", 1), ("d128", 0)] +
+                         [(name, 0) for name in sorted(LIBRARY)])
+def test_large_batch_step(name, shift):
     """More than 32 sequences: the same projections, positions per row, and the
-    LM head of 544 columns (17 groups of 32)."""
-    m = _model("d64", 64)
+    LM head of 544 columns (17 groups of 32; on the library's product where the
+    logits start `shift` floats past a 16-byte boundary)."""
+    m = _model(name, 64)
     ref = _Ref(m)
     rng = np.random.default_rng(5)
     B, n = 41, 21
-    note("prompt gemm: batched step of 41")
+    note(f"prompt gemm: batched step of 41, {name}, logits shifted by {shift}")
     ids = rng.integers(0, m.config.vocab_size, (B, n)).astype(np.int32)
     pool, p = _pages(m, 32 * B)
     bt = torch.from_numpy(rng.permutation(p).astype(np.int32).reshape(B, 2)).cuda()
@@ -125,7 +159,9 @@ def test_large_batch_step():
         m.prefill_paged(ids[b, :lens[b] - 1], pool, p, bt[b].contiguous(), 2)
     tok = torch.from_numpy(ids[np.arange(B), lens - 1]).cuda()
     ln = torch.from_numpy(lens).cuda()
-    logits = torch.empty((B, m.config.vocab_size), dtype=torch.float32, device="cuda")
+    size = B * m.config.vocab_size
+    buf = torch.full((size + 4,), 7.0, dtype=torch.float32, device="cuda")
+    logits = buf[shift:shift + size].view(B, -1)
     nxt = torch.empty(B, dtype=torch.int32, device="cuda")
     m.decode_paged(tok, pool, p, bt, 2, ln - 1, ln, 32, logits, nxt)
     torch.cuda.synchronize()
@@ -133,4 +169,5 @@ def test_large_batch_step():
         want, _ = ref.prompt(ids[b, :lens[b]])
         assert _rel(logits[b], want) < 4e-3, b
     assert torch.equal(nxt.long(), logits.argmax(1))
+    assert bool((buf[:shift] == 7).all()) and bool((buf[shift + size:] == 7).all())
     m.close()
