@@ -410,24 +410,32 @@ gemm_reduce_kernel(const float* part, f16* out, uint32_t chunks, int ranges) {
 
 // The tile for a shape: the smallest estimate over four tiles of rounds x
 // (start and end of a workgroup + steps x time of a step).  The step times (us)
-// were measured with few workgroups resident and with every slot taken, where
-// the L2 -> CU path is shared; between the two they are interpolated.
-// M x N x K in us on one box, tiles in the table's order, at 2048 rows:
-// gate/up 11264 x 2048 82.5 / 102 / 124 / 133, QKV 2560 x 2048 23.5 / 29.4 /
-// 30.7 / 33.6, o 2048 x 2048 21.2 / 18.9 / 23.2 / 24.3, down 2048 x 5632
-// 51.0 / 45.9 / 58.9 / 62.6; at 512 rows 24.3 / 29.1 / 32.7 / 34.9, 20.3 / 12.8 /
-// 9.8 / 11.3, 19.8 / 12.5 / 9.6 / 9.9, 48.6 / 32.9 / 25.1 / 22.2.
+// were measured on weights that no cache holds, as a model meets them (one set
+// after another, 700 MB in all): few workgroups resident, and every slot taken,
+// where the L2 -> CU path is shared; between the two they are interpolated, but
+// for the 64 x 64 tile, which shares a CU (and its path) from the 257th
+// workgroup on.  On warm weights the same steps take .50-.75, .28-.46, .19-.27 and
+// .21-.28, and a choice by those ran 320-700 rows on 128 x 64 tiles, slower than
+// rocBLAS.  Us in the table's order, then rocBLAS without the epilogue's work:
+//   rows   down 2048 x 5632           o 2048 x 2048              QKV 2560 x 2048
+//    320   74 / 45 / 40 / 29 | 29     28 / 18 / 16 / 13 | 13     31 / 20 / 17 / 14 | 13
+//    512   79 / 53 / 40 / 30 | 29     30 / 20 / 16 / 13 | 13     33 / 22 / 17 / 18 | 15
+//   1024   77 / 52 / 40 / 43 | 40     30 / 21 / 16 / 17 | 17     33 / 23 / 32 / 30 | 23
+//   2048   75 / 57 / 78 / 85 | 58     30 / 24 / 31 / 33 | 25     33 / 43 / 47 / 47 | 29
+// gate/up 11264 x 2048: 33 rows 29 / 20 / 19 / 16 | 16, 256 33 / 24 / 33 / 36 | 28,
+// 512 34 / 43 / 47 / 51 | 32, 2048 102 / 126 / 163 / 174 | 88.
 struct GemmTile {
     int bn, bm, slots;
     float lo, hi;
 };
 constexpr GemmTile kTiles[] = {
-    {256, 128, 256, 0.50f, 0.75f},
-    {128, 128, 256, 0.28f, 0.46f},
-    {128, 64, 256, 0.19f, 0.27f},
-    {64, 64, 512, 0.21f, 0.28f},
+    {256, 128, 256, 0.80f, 1.00f},
+    {128, 128, 256, 0.46f, 0.62f},
+    {128, 64, 256, 0.40f, 0.42f},
+    {64, 64, 512, 0.30f, 0.45f},
 };
 constexpr float kTileEnds = 3.f;   // us: first loads, epilogue
+constexpr int kNumCUs = 256;
 
 int gemm_pick(int M, int N, int K) {
     int best = 0;
@@ -437,7 +445,9 @@ int gemm_pick(int M, int N, int K) {
         const int64_t T = (int64_t)((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm);
         const int64_t rounds = (T + c.slots - 1) / c.slots;
         const float full = std::min(1.f, static_cast<float>(T) / static_cast<float>(c.slots));
-        const float step = c.lo + (c.hi - c.lo) * std::max(0.f, (full - 0.25f) / 0.75f);
+        const float share = c.slots > kNumCUs ? (T > kNumCUs ? 1.f : 0.f)
+                                              : std::max(0.f, (full - 0.25f) / 0.75f);
+        const float step = c.lo + (c.hi - c.lo) * share;
         const float t = static_cast<float>(rounds) * (kTileEnds + step * static_cast<float>(K / 64));
         if (i == 0 || t < cost) {
             cost = t;
