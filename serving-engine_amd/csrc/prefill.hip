@@ -76,8 +76,9 @@ struct PrefillArgs {
     int paired;             // 1: query blocks i and n-1-i share a workgroup (two passes)
     float scale_log2;
     int HG, nsub;           // SUB: query heads per workgroup, workgroups per KV head
-    int fold;               // unpaired: the longer half of the blocks longest first, then the
-                            // shorter half shortest first (two workgroups per CU)
+    int fold;               // unpaired, > 0: this many blocks longest first, then the others
+                            // shortest first (two workgroups per CU)
+    int side;               // fold: the blocks of one rank of all sequences side by side
     // CACHED: the q rows sit at positions first .. first + S - 1 and all keys are
     // read from the pages (k, v: the pools; bt, max_pages, num_pages as above).
     int first;
@@ -231,8 +232,12 @@ prefill_mfma_kernel(const PrefillArgs a) {
     const int hw = SUB ? a.Hkv * a.nsub : a.Hkv;   // workgroups per block or pair
     const int kvh = SUB ? blockIdx.x % hw / a.nsub : blockIdx.x % a.Hkv;
     const int sub = SUB ? blockIdx.x % hw % a.nsub : 0;
-    const int pair = blockIdx.x / hw;   // pair index (paired) or block rank, longest first
-    const int b = blockIdx.y;
+    // pair index (paired) or block rank, longest first, and sequence; side by side:
+    // grid (KV head, group and sequence, 1, block)
+    const bool side = D == 64 && KG == 2 && !CACHED && a.side;
+    const int xq = blockIdx.x / hw;
+    const int pair = side ? blockIdx.z : xq;
+    const int b = side ? xq : blockIdx.y;
     const int S = a.S;
     const int G = SUB ? min(a.HG, a.G - sub * a.HG) : a.G;   // this workgroup's query heads
     const int head0 = kvh * a.G + sub * a.HG;                // and the first of them
@@ -341,7 +346,7 @@ prefill_mfma_kernel(const PrefillArgs a) {
             if (pass == 1) break;
             qblk = a.n_qblk - 1 - pair;   // one block per workgroup, longest first
             if (D == 64 && KG == 2)
-                if (a.fold && pair >= (a.n_qblk + 1) / 2) qblk = pair - (a.n_qblk + 1) / 2;
+                if (a.fold && pair >= a.fold) qblk = pair - a.fold;
         }
         const int q0 = qblk * BM;
 
@@ -908,14 +913,23 @@ int prefill_impl(const void* q, const void* k, const void* v, void* out, int64_t
         const int64_t pgrid = (int64_t)hkv * a.nsub * ((a.n_qblk + 1) / 2) * batch;
         a.paired = (pgrid >= kNumCUs) ? 1 : 0;
         // D = 64 at KG = 2 keeps two workgroups on a CU (64 KB LDS, 125 VGPRs):
-        // while every block is resident at once, a block each, the long half
-        // ahead of the short half in reverse, so that a CU's two add up alike
-        // (32/8 heads 2048 34.5 paired / 32.6, 32/4 heads 33.1 / 31.8).
-        if (d == 64 && kg == 2 && (int64_t)hkv * a.nsub * a.n_qblk * batch <= 2 * kNumCUs) {
+        // while every block is resident at once, a block each, as many of the
+        // longest as there are CUs longest first, then the others shortest first,
+        // so that a CU's two add up alike (32/8 heads 2048 34.5 paired / 32.6, 32/4
+        // heads 33.1 / 31.8).  A batch goes block by block, its sequences side by
+        // side: one sequence after another a CU met two long blocks (32/8 heads,
+        // 2 x 1000 26.7 / 21.3, paired 22.5; 3 x 333 11.6 / 10.4, paired 10.5; 4 x
+        // 512 18.2 / 15.0, paired 17.0).
+        const int64_t side = (int64_t)hkv * a.nsub * batch;   // workgroups per block rank
+        const int blocks = a.paired ? (a.n_qblk + 1) / 2 : a.n_qblk;
+        dim3 grid(hkv * a.nsub * blocks, batch);
+        if (d == 64 && kg == 2 && side * a.n_qblk <= 2 * kNumCUs) {
             a.paired = 0;
-            a.fold = 1;
+            a.fold = std::max(1, static_cast<int>(kNumCUs / side));
+            a.side = batch > 1;
+            grid = a.side ? dim3(static_cast<unsigned>(side), 1, a.n_qblk)
+                          : dim3(hkv * a.nsub * a.n_qblk);
         }
-        dim3 grid(hkv * a.nsub * (a.paired ? (a.n_qblk + 1) / 2 : a.n_qblk), batch);
         const dim3 blk(8 * kWave);
         auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, grid, blk, 0, s, a); };
         if (d == 64)

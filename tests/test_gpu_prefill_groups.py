@@ -35,6 +35,20 @@ def _reference(q, k, v):
 @pytest.mark.parametrize("s,batch", [(1, 2), (31, 1), (33, 1), (64, 3), (65, 1), (96, 1), (500, 1),
                                      (777, 2)])
 def test_head_groups(hq, hkv, d, s, batch):
+    _check_prefill(hq, hkv, d, s, batch)
+
+
+@pytest.mark.parametrize("hq,hkv,s,batch", [(8, 4, 500, 16), (8, 4, 300, 25), (16, 2, 333, 9),
+                                            (5, 1, 260, 33), (2, 2, 250, 61), (4, 2, 20, 40),
+                                            (7, 1, 31, 120), (32, 8, 333, 3)])
+def test_folded_batches(hq, hkv, s, batch):
+    """Batches whose blocks are all resident at once, two on a CU: every block of
+    every sequence once, with more and with fewer workgroups of one rank than CUs
+    and a single block a sequence."""
+    _check_prefill(hq, hkv, 64, s, batch)
+
+
+def _check_prefill(hq, hkv, d, s, batch):
     note(f"prefill groups {hq}/{hkv}x{d} S={s} B={batch}")
     torch.manual_seed(s + hq)
     q = torch.randn(batch, s, hq, d, device="cuda").half()
