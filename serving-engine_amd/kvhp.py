@@ -224,19 +224,38 @@ def _ptr(t) -> Optional[int]:
     return t.data_ptr()
 
 
+_raw_stream = None    # torch's (device index) -> current stream's handle, once a call was made
+_raw_device = None    # and its current device's index
+
+
+def _first_stream() -> int:
+    """torch's current stream, through torch's own initialisation of the device
+    (and its refusal of forked children); later calls take the handle without
+    building a torch.cuda.Stream object around it (0.2 against 2.8 us, a third of
+    a small call's host time)."""
+    global _raw_stream, _raw_device
+    import torch   # here: importing this module loads no torch
+    handle = torch.cuda.current_stream().cuda_stream
+    _raw_device = getattr(torch._C, "_cuda_getDevice", None)   # not public names
+    if _raw_device is not None:
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return handle
+
+
+def _forget_stream() -> None:
+    global _raw_stream
+    _raw_stream = None
+
+
+os.register_at_fork(after_in_child=_forget_stream)
+
+
 def _stream(stream) -> Optional[int]:
     if stream is not None:
         return stream.cuda_stream
-    import torch   # here, so that importing this module loads no torch
-    # The current stream's handle without building a torch.cuda.Stream object
-    # around it (0.4 against 2.8 us, a third of a small call's host time), once
-    # torch has initialised the device (never in a forked child, which it refuses).
-    if torch.cuda.is_initialized():
-        try:
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
-        except AttributeError:   # not public names
-            pass
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None:
+        return _first_stream()
+    return _raw_stream(_raw_device())
 
 
 # ----------------------------------------------------------------- views --

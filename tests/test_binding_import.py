@@ -35,6 +35,14 @@ def test_default_stream_is_the_current_one():
             "assert not torch.cuda.is_initialized(); h = kvhp._stream(None); "
             "assert torch.cuda.is_initialized() and h == torch.cuda.current_stream().cuda_stream")
     subprocess.run([sys.executable, "-c", code], check=True)
+    code = (f"import os, sys; sys.path.insert(0, {PKG!r}); import kvhp, torch; kvhp._stream(None)\n"
+            "r, w = os.pipe()\n"
+            "if os.fork() == 0:\n"
+            "    try: kvhp._stream(None)\n"
+            "    except RuntimeError as e: os.write(w, str(e).encode())\n"
+            "    os._exit(0)\n"
+            "os.close(w); os.wait(); sys.exit(0 if b'fork' in os.read(r, 4096) else 1)")
+    subprocess.run([sys.executable, "-c", code], check=True)   # a forked child is refused
     side = torch.cuda.Stream()
     assert kvhp._stream(None) == torch.cuda.current_stream().cuda_stream
     with torch.cuda.stream(side):
