@@ -84,10 +84,10 @@ __device__ __forceinline__ float r16(float v) { return static_cast<float>(static
 // product (g has 11 bits, the constant's head 13) plus the rest of the constant;
 // the quotient is a reciprocal's product and one residual step, in sixteenths so
 // that no reciprocal is subnormal.  Where the residual is zero, or NaN (infinite
-// gates and exponentials), the product stands.  A 2048-id prompt of the 22-layer
-// 2048 / 5632 model takes 5508 us, and 2.7 % (against 1.4 %) over that of
-// v_exp_f32 of the rounded product and v_rcp_f32 with expf and the IEEE division;
-// those two alone are up to 61 units of 2^-24 off, expf and this 2.4.
+// gates and exponentials), the product stands.  v_exp_f32 of the rounded product
+// and v_rcp_f32 are up to 61 units of 2^-24 off, expf and this 2.4; a 2048-id
+// prompt of the 22-layer 2048 / 5632 model takes 1.1-1.4 % longer than with those
+// two (5500 against 5440 us), and 2.7 % with expf and the IEEE division.
 __device__ __forceinline__ float silu_mul(float g, float u) {
     constexpr float hi = -1.442626953125f, lo = static_cast<float>(-1.4426950408889634 - hi);
     const float gc = __builtin_amdgcn_fmed3f(g, -200.f, 200.f);   // exp(-g) infinite or 0 beyond
